@@ -72,15 +72,19 @@ int qx_device_is_gfx950(void);
  * 31: config 30's arithmetic on 256x320 tiles (N a multiple of 320): each
  *     wave's 160 weight rows lie in two 128-row scale blocks and each of
  *     its 16-row tiles is promoted with its block's scale; bit-identical
- *     to config 30 where N is a multiple of both.
+ *     to config 30 where N is a multiple of both;
+ * 40-47: config 30's arithmetic, bit-identical to it, on smaller tiles for
+ *     few token rows, one workgroup per tile (N a multiple of the tile's
+ *     weights): 40: 16x32, 41: 32x32, 42: 64x64, 43: 128x64, 44: 192x64,
+ *     45: 128x128, 46: 192x128, 47: 256x128.
  * Configs 10, 11, 12 and 22 rescale the accumulators in place
  * (acc *= s_prev / s per block, the last s in the epilogue) and compute
  * each element with the same operations in the same order: their results
  * are bit-identical for finite operands. A weight block whose scale is 0
  * is skipped by 10, 11 and 22 and run on zeroed weight rows by 12, so a
  * NaN activation code in such a block gives 0 under 10/11/22 and NaN under
- * 12; configs 30 and 31 add 0 * partial, NaN as well, as DeepGEMM's
- * promotion does. Configs 30 and 31 sum in another order (within the bf16
+ * 12; the promotion configs (30, 31, 40-47) add 0 * partial, NaN as well,
+ * as DeepGEMM's promotion does. They sum in another order (within the bf16
  * tolerance of the others and of the dequantized product); a caller that
  * needs a row's result independent of M picks the family by N alone.
  */
@@ -183,7 +187,8 @@ int qx_silu_mul_quant(const void* gate_up, int64_t gu_ld, void* q, int64_t q_ld,
  * qx_silu_mul_quant; the bf16 gate_up rows are never written. config: 10
  * (one workgroup per 256x256 tile) or 22 (persistent, as config 22 of
  * qx_gemm_fp8_blockscaled), the same bits as configs 10-22; 30 (the
- * promotion form, as config 30 of qx_gemm_fp8_blockscaled).
+ * promotion form, as config 30 of qx_gemm_fp8_blockscaled) or 48, 49, 50
+ * (the same bits on 64, 96 or 128 tokens x 256 weights, for few token rows).
  */
 int qx_gemm_fp8_swiglu_quant(const void* A, const float* sA, const void* W, const float* sW,
                              void* Q, int64_t q_ld, float* Qs, int64_t qs_ld, int64_t M,

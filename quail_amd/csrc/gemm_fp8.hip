@@ -36,6 +36,7 @@
 //     L2) runs a contiguous band of tiles that share operands.
 #include <type_traits>
 
+#include "gemm_small.h"
 #include "qx_common.h"
 #include "qx_status.h"
 
@@ -1465,6 +1466,51 @@ int launch_promo(const void* A, const float* sA, const void* W, const float* sW,
                      ldc, sa_ld, tiles_m, tiles_n, 4, (uint8_t*)Q, q_ld, Qs, qs_ld);
   QX_LAUNCH_STATUS();
 }
+// one tile of gemm_small.h per workgroup
+template <int BM, int BN, int WM, int WN, int STAGES, int KPB, bool SWIGLU>
+int launch_ring(const void* A, const float* sA, const void* W, const float* sW, void* C, int M,
+                int N, int K, int64_t lda, int64_t ldc, int64_t sa_ld, void* Q, int64_t q_ld,
+                float* Qs, int64_t qs_ld, hipStream_t stream) {
+  const int tiles_m = (M + BM - 1) / BM;
+  const int tiles_n = N / BN;
+  QX_CHECK(N % BN == 0, "gemm: N=%d is not a multiple of the tile's %d", N, BN);
+  QX_CHECK((int64_t)tiles_m * tiles_n < (1LL << 31) / (64 * WM * WN),
+           "gemm: %d x %d tiles exceed the grid", tiles_m, tiles_n);
+  hipLaunchKernelGGL((gemm_fp8_promo_ring_kernel<BM, BN, WM, WN, STAGES, KPB, SWIGLU>),
+                     dim3(tiles_m * tiles_n), dim3(64 * WM * WN), 0, stream, (const uint8_t*)A,
+                     sA, (const uint8_t*)W, sW, (uint16_t*)C, M, N, K, lda, ldc, sa_ld, tiles_m,
+                     tiles_n, (uint8_t*)Q, q_ld, Qs, qs_ld);
+  QX_LAUNCH_STATUS();
+}
+
+// configs 40-47 (plain) and 48-50 (SwiGLU): false if `config` is none of them
+bool small_config(int config, bool swiglu) {
+  return swiglu ? config >= 48 && config <= 50 : config >= 40 && config <= 47;
+}
+
+int launch_small(int config, const void* A, const float* sA, const void* W, const float* sW,
+                 void* C, int M, int N, int K, int64_t lda, int64_t ldc, int64_t sa_ld, void* Q,
+                 int64_t q_ld, float* Qs, int64_t qs_ld, hipStream_t stream) {
+#define QX_RING(CODE, BM, BN, WM, WN, ST, KPB, SG)                                              \
+  case CODE:                                                                                   \
+    return launch_ring<BM, BN, WM, WN, ST, KPB, SG>(A, sA, W, sW, C, M, N, K, lda, ldc, sa_ld, \
+                                                    Q, q_ld, Qs, qs_ld, stream);
+  switch (config) {
+    QX_RING(40, 16, 32, 1, 2, 4, 4, false)
+    QX_RING(41, 32, 32, 2, 2, 4, 2, false)
+    QX_RING(42, 64, 64, 4, 2, 4, 2, false)
+    QX_RING(43, 128, 64, 4, 2, 4, 1, false)
+    QX_RING(44, 192, 64, 4, 2, 4, 1, false)
+    QX_RING(45, 128, 128, 4, 2, 4, 1, false)
+    QX_RING(46, 192, 128, 4, 2, 3, 1, false)
+    QX_RING(47, 256, 128, 4, 2, 3, 1, false)
+    QX_RING(48, 64, 256, 2, 4, 3, 1, true)
+    QX_RING(49, 96, 256, 2, 4, 3, 1, true)
+    QX_RING(50, 128, 256, 2, 4, 3, 1, true)
+  }
+#undef QX_RING
+  return QX_EINVAL;  // not reached: small_config
+}
 }  // namespace
 }  // namespace qx
 
@@ -1479,7 +1525,11 @@ extern "C" {
 // persistent grid with the K pipeline running across tiles (falls back to
 // 10 when there are too few tiles or an odd number of 128-K blocks). The
 // promotion family, bit-identical to each other: 30 (256 x 256 tiles) and
-// 31 (256 x 320 tiles), both persistent.
+// 31 (256 x 320 tiles), both persistent, and the smaller tiles of
+// gemm_small.h, one workgroup each: 40: 16 x 32, 41: 32 x 32, 42: 64 x 64,
+// 43: 128 x 64, 44: 192 x 64, 45: 128 x 128, 46: 192 x 128, 47: 256 x 128
+// (tokens x weights; any N they divide); with the SiLU-quant epilogue 48:
+// 64 x 256, 49: 96 x 256, 50: 128 x 256.
 // gate_up projection + SiLU-gated product + per-128 FP8 quant in one launch:
 // W / sW are the gate_up weight (2I x K, rows [gate | up]) and its scales;
 // I = intermediate width.
@@ -1498,9 +1548,12 @@ int qx_gemm_fp8_swiglu_quant(const void* A, const float* sA, const void* W, cons
   QX_CHECK(qs_ld >= M && sa_ld >= M, "gemm_swiglu: scale strides");
   QX_CHECK(M < (1LL << 31) && 2 * I < (1LL << 31) && K < (1LL << 31), "gemm_swiglu: dims");
   QX_CHECK(((uintptr_t)A & 15) == 0 && ((uintptr_t)W & 15) == 0, "gemm_swiglu: alignment");
-  QX_CHECK(config == 10 || config == 22 || config == 30,
-           "gemm_swiglu: config %d (10, 22 or 30)", config);
+  QX_CHECK(config == 10 || config == 22 || config == 30 || qx::small_config(config, true),
+           "gemm_swiglu: config %d (10, 22, 30 or 48-50)", config);
   if (M == 0) return QX_OK;
+  if (qx::small_config(config, true))
+    return qx::launch_small(config, A, sA, W, sW, nullptr, (int)M, (int)(2 * I), (int)K, lda, 0,
+                            sa_ld, Q, q_ld, Qs, qs_ld, stream);
   if (config == 30) {
     QX_CHECK(256 * lda < (1LL << 32) && (I + 128) * K < (1LL << 32),
              "gemm_swiglu config 30: a tile's rows must span less than 4 GiB (lda=%lld, K=%lld)",
@@ -1532,6 +1585,9 @@ int qx_gemm_fp8_blockscaled(const void* A, const float* sA, const void* W, const
   QX_CHECK(((uintptr_t)C & 7) == 0, "gemm: C not 8-byte aligned");
   if (M == 0) return QX_OK;
   const int m = (int)M, n = (int)N, k = (int)K;
+  if (qx::small_config(config, false))
+    return qx::launch_small(config, A, sA, W, sW, C, m, n, k, lda, ldc, sa_ld, nullptr, 0,
+                            nullptr, 0, stream);
   switch (config) {
     case 10:
       QX_CHECK(n % 256 == 0, "gemm config 10 needs N %% 256 == 0 (N=%d)", n);
@@ -1565,7 +1621,7 @@ int qx_gemm_fp8_blockscaled(const void* A, const float* sA, const void* W, const
       return qx::launch_promo<false, 320>(A, sA, W, sW, C, m, n, k, lda, ldc, sa_ld, nullptr, 0,
                                           nullptr, 0, stream);
     default:
-      QX_CHECK(false, "gemm: unknown config %d (10, 11, 12, 22, 30 or 31)", config);
+      QX_CHECK(false, "gemm: unknown config %d (10, 11, 12, 22, 30, 31 or 40-47)", config);
   }
 }
 

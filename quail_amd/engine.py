@@ -16,6 +16,7 @@ Layouts are the reference's: FP8 activations are e4m3fn (n, K) with
 (N/128, K/128).
 """
 
+import functools
 import os
 
 import torch
@@ -29,7 +30,8 @@ GROUP = 128
 # one 16x16x128 MFMA and promoted into an fp32 total, total += (sA * sW) *
 # partial (DeepGEMM's form), persistent grids; 30 = 256 tokens x 256
 # weights, 31 = 256 x 320 (widths that are multiples of 320: whole waves
-# where N = 2560 makes 2.5 or 1.25 waves of 256 x 256 tiles). Rescale family
+# where N = 2560 makes 2.5 or 1.25 waves of 256 x 256 tiles); 40-47 the same
+# arithmetic on smaller tiles (PROMOTION_TILES). Rescale family
 # (10, 11, 12, 22): the MFMA accumulators rescaled in place by s_prev / s at
 # each block; 10 = 256 x 256, one workgroup per tile; 11 = 256 x 128 (widths
 # not a multiple of 256); 22 = config 10's tiles on a persistent grid; 12 =
@@ -41,7 +43,7 @@ GROUP = 128
 # takes the promotion family, the rest config 11. QUAIL_GEMM_CONFIG forces
 # one.
 GEMM_CONFIG_ENV = "QUAIL_GEMM_CONFIG"
-GEMM_CONFIGS = (10, 11, 12, 22, 30, 31)
+GEMM_CONFIGS = (10, 11, 12, 22, 30, 31) + tuple(range(40, 48))
 RESCALE_CONFIGS = (10, 11, 12, 22)
 PROMOTION_CONFIGS = (30, 31)
 GEMM_PROMOTION_CONFIG = 30
@@ -92,19 +94,67 @@ def _wide_tiles_fill_better(n: int, m: int) -> bool:
                                                  else float("inf"))
 
 
+# The promotion family's tiles: config -> (tokens, weights, workgroups at a
+# time, us per 128-K block, us besides). A launch takes about
+#   rounds x (us besides + K / 128 x us per block)
+# with rounds = tiles over workgroups at a time, rounded up (a CU holds one
+# workgroup, of 32 x 32 tiles two). The times are measured on one MI355X over
+# the Qwen3-4B, -8B and -32B projections at 1 to 8192 rows (launches of 60 to
+# 256 tiles, weights not in L2); choosing by them lost 0.1% on average, and
+# 7% at most, against the fastest tile of each of those 348 launches.
+PROMOTION_TILES = {
+    40: (16, 32, 256, 0.167, 2.9), 41: (32, 32, 512, 0.220, 3.4),
+    42: (64, 64, 256, 0.302, 3.8), 43: (128, 64, 256, 0.442, 4.3),
+    44: (192, 64, 256, 0.539, 4.6), 45: (128, 128, 256, 0.602, 6.3),
+    46: (192, 128, 256, 0.781, 7.0), 47: (256, 128, 256, 0.979, 7.9),
+    30: (256, 256, 256, 1.443, 3.9), 31: (256, 320, 256, 1.686, 10.0),
+}
+# the same with the SiLU-quant epilogue
+SWIGLU_TILES = {48: (64, 256, 256, 1.369, -4.0), 49: (96, 256, 256, 1.380, -0.5),
+                50: (128, 256, 256, 1.426, 0.2), 30: (256, 256, 256, 1.933, 1.7)}
+SWIGLU_SMALL_CONFIGS = (48, 49, 50)
+
+
+@functools.lru_cache(maxsize=4096)
+def _fastest_tile(n: int, k: int, m: int, swiglu: bool, large: int) -> int:
+    """The tile config of an (m x k) by (n x k) promotion GEMM: `large` (30
+    or 31) unless a smaller tile's measured cost is below its. A row's bits
+    are the same under all of them."""
+    best, cost = large, None
+    for config, (bm, bn, at_once, block, rest) in (SWIGLU_TILES if swiglu
+                                                   else PROMOTION_TILES).items():
+        if n % bn or (config in PROMOTION_CONFIGS and config != large):
+            continue
+        rounds = -(-(-(-m // bm) * (n // bn)) // at_once)
+        c = rounds * (rest + k // GROUP * block)
+        if cost is None or c < cost:
+            best, cost = config, c
+    return best
+
+
+def gemm_tiles(n: int, k: int, m: int) -> int:
+    """The config Engine.gemm launches: gemm_config's, and within the
+    promotion family the tile that takes least time at m rows."""
+    config = gemm_config(n, k, m)
+    if config not in PROMOTION_CONFIGS or GEMM_CONFIG_ENV in os.environ:
+        return config
+    return _fastest_tile(n, k, m, False, config)
+
+
 SWIGLU_CONFIG_ENV = "QUAIL_SWIGLU_CONFIG"
 
 
 def swiglu_config(n: int = 0, k: int = 0, m: int = 0) -> int:
     """Tile schedule of the gate_up GEMM with the SiLU-quant epilogue (n =
-    gate_up rows, 256 per tile): the promotion kernel (30) for every shape;
-    10 and 22 (the rescale family) stay selectable. QUAIL_SWIGLU_CONFIG
-    forces it alone, QUAIL_GEMM_CONFIG with every GEMM."""
+    gate_up rows, 256 per tile): the promotion form, on the tile that takes
+    least time at m rows (30's 256 x 256 for packs); 10 and 22 (the rescale
+    family) stay selectable. QUAIL_SWIGLU_CONFIG forces it alone,
+    QUAIL_GEMM_CONFIG with every GEMM."""
     for env in (SWIGLU_CONFIG_ENV, GEMM_CONFIG_ENV):
         forced = os.environ.get(env)
-        if forced is not None and int(forced) in (10, 22, 30):
+        if forced is not None and int(forced) in (10, 22, 30) + SWIGLU_SMALL_CONFIGS:
             return int(forced)
-    return SWIGLU_DEFAULT_CONFIG
+    return _fastest_tile(n, k, m, True, SWIGLU_DEFAULT_CONFIG)
 
 
 class Engine:
@@ -186,7 +236,7 @@ class Engine:
             start.record()
         _lib.call("qx_gemm_fp8_blockscaled", _ptr(q_input), _ptr(input_scale), _ptr(w),
                   _ptr(sw), _ptr(out), m, n, k, q_input.stride(0), out.stride(0),
-                  self._scale_ld(input_scale), gemm_config(n, k, m), _stream())
+                  self._scale_ld(input_scale), gemm_tiles(n, k, m), _stream())
         if timed:
             end.record()
             self.gemm_timer.append((m, n, k, start, end, False))

@@ -211,6 +211,66 @@ def test_gemm_wide_promotion_tiles_at_widths_only_320_divides(m, n, k, monkeypat
     _bf16_close(_run_gemm(q, s, wq, ws), ref.gemm(q, s, ref.RefLinear(wq, ws)))
 
 
+SMALL_TILES = {40: (16, 32), 41: (32, 32), 42: (64, 64), 43: (128, 64), 44: (192, 64),
+               45: (128, 128), 46: (192, 128), 47: (256, 128)}
+
+
+@pytest.mark.parametrize("config", sorted(SMALL_TILES))
+@pytest.mark.parametrize("k", [128, 256, 384, 640, 1152, 2176])
+def test_gemm_small_promotion_tiles_equal_config_30(config, k, monkeypatch):
+    """Configs 40-47 (config 30's arithmetic on smaller tiles, one workgroup
+    each) give config 30's bits: one row, a row less and a row more than the
+    tile, several token tiles; one to 17 128-K blocks (fewer than the ring's
+    stages, groups of two and four blocks with a partial last one)."""
+    bm, _ = SMALL_TILES[config]
+    n = 1280
+    q, s, wq, ws = _gemm_case(2 * bm + 5, n, k, seed=config + k)
+    ws[3, 0] = 0.0
+    monkeypatch.setenv("QUAIL_GEMM_CONFIG", str(PROMOTION_CONFIG))
+    want = _run_gemm(q, s, wq, ws)
+    monkeypatch.setenv("QUAIL_GEMM_CONFIG", str(config))
+    for m in (1, bm - 1, bm + 1, 2 * bm + 5):
+        got = _run_gemm(q[:m], s[:m], wq, ws)
+        assert torch.equal(got.view(torch.int16), want[:m].view(torch.int16)), m
+
+
+@pytest.mark.parametrize("config", [48, 49, 50])
+@pytest.mark.parametrize("m,i,k", [(1, 256, 128), (63, 384, 256), (97, 1280, 384),
+                                   (300, 768, 1152)])
+def test_gate_up_swiglu_quant_small_tiles_equal_config_30(config, m, i, k, monkeypatch):
+    """Configs 48-50 (64, 96 and 128 tokens x 256 gate_up rows) give the codes
+    and scales of config 30: one row, partial token tiles, one to nine
+    128-K blocks."""
+    eng = _engine()
+    q, s, wq, ws = _gemm_case(m, 2 * i, k, seed=m + i + k)
+    lin = type("L", (), {})()
+    lin.weight, lin.weight_scale_inv = wq.to(DEV), ws.to(DEV)
+    scales = torch.empty((k // 128, m), dtype=torch.float32, device=DEV)
+    scales.copy_(s.T)
+    outs = {}
+    for c in (30, config):
+        monkeypatch.setenv("QUAIL_SWIGLU_CONFIG", str(c))
+        outs[c] = eng.gate_up_activation_quant(q.to(DEV), scales.permute(1, 0), lin)
+    assert torch.equal(outs[30][0].view(torch.uint8), outs[config][0].view(torch.uint8))
+    assert torch.equal(outs[30][1], outs[config][1])
+
+
+def test_gemm_rows_do_not_depend_on_the_tile_the_row_count_takes(monkeypatch):
+    """A row's bits are the same however many rows share the launch, over the
+    tiles the engine picks at 1 to 5000 rows."""
+    from quail_amd.engine import gemm_tiles
+    monkeypatch.delenv("QUAIL_GEMM_CONFIG", raising=False)
+    n, k = 2560, 640
+    q, s, wq, ws = _gemm_case(5000, n, k, seed=5)
+    want = _run_gemm(q, s, wq, ws)
+    picked = {gemm_tiles(n, k, 5000)}
+    for m in (1, 40, 300, 500, 700, 1100, 1500, 2400):
+        picked.add(gemm_tiles(n, k, m))
+        assert torch.equal(_run_gemm(q[:m], s[:m], wq, ws).view(torch.int16),
+                           want[:m].view(torch.int16)), m
+    assert len(picked) >= 6, picked
+
+
 def test_gemm_configs_agree_with_zero_weight_blocks(monkeypatch):
     """Weight blocks whose scale is 0 add nothing; configurations skip them
     or run them on zero fragments, and all must agree bit for bit: zero

@@ -128,6 +128,32 @@ def test_gemm_family_depends_on_width_only():
         assert len(fams) == 1, n
 
 
+def test_promotion_tiles_divide_the_width_and_stay_in_the_family(monkeypatch):
+    """The tile the engine launches at any row count: one whose weights divide
+    N, of the promotion family exactly where gemm_config is; small for few
+    rows, config 30 or 31 for packs; the environment variable forces one."""
+    from quail_amd import engine as e
+    monkeypatch.delenv(e.GEMM_CONFIG_ENV, raising=False)
+    monkeypatch.delenv(e.SWIGLU_CONFIG_ENV, raising=False)
+    rows = (1, 15, 16, 17, 46, 97, 255, 333, 1003, 2048, 3600, 8192, 16294, 32768)
+    for n in (256, 640, 1280, 1920, 2560, 4096, 5120, 6144, 10240, 2688):
+        for k in (128, 2560, 9728, 25600):
+            for m in rows:
+                config = e.gemm_tiles(n, k, m)
+                if e.gemm_config(n, k, m) == e.GEMM_ODD_WIDTH_CONFIG:
+                    assert config == e.GEMM_ODD_WIDTH_CONFIG
+                else:
+                    assert n % e.PROMOTION_TILES[config][1] == 0
+    for m in rows:
+        assert e.swiglu_config(19456, 2560, m) in e.SWIGLU_TILES
+    assert e.gemm_tiles(2560, 9728, 46) == 40
+    assert e.gemm_tiles(2560, 9728, 16294) == 31
+    assert e.gemm_tiles(6144, 2560, 16294) == 30
+    assert e.swiglu_config(19456, 2560, 46) == 48
+    monkeypatch.setenv(e.GEMM_CONFIG_ENV, "30")
+    assert e.gemm_tiles(2560, 9728, 46) == 30
+
+
 def test_swiglu_config_choice_by_shape(monkeypatch):
     from quail_amd.engine import GEMM_CONFIG_ENV, SWIGLU_CONFIG_ENV, swiglu_config
     monkeypatch.delenv(GEMM_CONFIG_ENV, raising=False)
