@@ -797,6 +797,52 @@ def test_paged_attention_32_row_workgroups_are_bit_identical(v_dtype):
                                atol=2e-2)
 
 
+@pytest.mark.parametrize("rows", [0, 32])
+@pytest.mark.parametrize("v_dtype", V_DTYPES)
+def test_paged_attention_around_its_tile_counts(rows, v_dtype):
+    """Sequences of zero to seven 64-key tiles, each with its last tile whole,
+    one key short and one key over (the pipeline's steps with loads spread
+    over the MFMAs take whole tiles only, three ahead; the last steps take
+    the rest), with one query row and with more rows than a workgroup holds:
+    exact fp32 attention, at both workgroup heights."""
+    from quail_amd.chunk import _work_list
+    from quail_amd import _lib
+
+    hq, hk, d, page = 32, 8, 128, 16
+    used, q_lens = [], []
+    for tiles in range(1, 8):
+        for keys in (64 * tiles - 1, 64 * tiles, 64 * tiles + 1):
+            for q_len in (1, min(keys, 67)):
+                used.append(keys)
+                q_lens.append(q_len)
+    rng = np.random.default_rng(17)
+    pages = [-(-u // page) for u in used]
+    perm = rng.permutation(sum(pages) + 9)
+    table = np.zeros((len(used), max(pages)), dtype=np.int32)
+    at = 0
+    for s_, need in enumerate(pages):
+        table[s_, :need] = perm[at:at + need]
+        at += need
+    g = _gen(18)
+    kp = torch.randn(len(perm) * page, hk, d, generator=g).to(torch.bfloat16)
+    vp = torch.randn(len(perm) * page, hk, d, generator=g).to(torch.bfloat16)
+    cu = np.concatenate([[0], np.cumsum(q_lens)]).astype(np.int32)
+    used = np.asarray(used, dtype=np.int32)
+    q = torch.randn(int(cu[-1]), hq, d, generator=g).to(torch.bfloat16)
+    want = ref.paged_attention(q, kp, vp, cu, used, table, page)
+    host = dict(cu_q=cu, used=used, causal=True)
+    work, n_work, picked = _work_list(host, (hq, hk, d), choose_rows=rows == 32)
+    assert picked == rows
+    dev = [torch.tensor(x, device=DEV) for x in (cu, used, table, work)]
+    kd, vd, q3 = kp.to(DEV), vp.to(v_dtype).to(DEV), q.to(DEV)
+    o = torch.full((q.shape[0], hq * d), float("nan"), dtype=torch.bfloat16, device=DEV)
+    _lib.call("qx_paged_attention", _ptr(q3), hq * d, _ptr(kd), _ptr(vd), _ptr(dev[0]),
+              _ptr(dev[1]), _ptr(dev[2]), dev[2].stride(0), len(used), int(max(q_lens)),
+              int(used.max()), hq, hk, d, page, float(d ** -0.5), 1, _ptr(o), None, o.stride(0),
+              None, 0, _ptr(dev[3]), n_work, rows, int(v_dtype == torch.bfloat16), _stream())
+    torch.testing.assert_close(o.float().cpu().view_as(want), want.float(), rtol=2e-2, atol=2e-2)
+
+
 @pytest.mark.parametrize("cache_dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("v_dtype", V_DTYPES)
 def test_attention_with_q_norm_on_load_is_bit_identical(cache_dtype, v_dtype):
