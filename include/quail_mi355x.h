@@ -317,10 +317,11 @@ int qx_paged_attention_qnorm(const void* q, int64_t q_ld, const void* k_pool, co
 
 /*
  * Host function: the query rows per workgroup (work-list tile height) that a
- * paged call over these sequences runs best with: 32 where qx_paged_attention
- * accepts it and the default-height work items read at most 8 64-key tiles
- * on average (short documents: two 4-wave workgroups per CU hide each
- * other's fixed cost), else the default. cu_q and used are host copies.
+ * paged or LSE call over these sequences runs best with: 32 where
+ * qx_paged_attention accepts it and the default-height work items read at
+ * most 8 64-key tiles on average (short documents: two 4-wave workgroups per
+ * CU hide each other's fixed cost), or many of them are half empty, or their
+ * workgroups do not outnumber the CUs; else the default. cu_q and used are host copies.
  * Returns the rows or -1. No reference counterpart (FlashAttention's varlen
  * grid has one tile height).
  */
@@ -365,6 +366,19 @@ int qx_attention_lse(const void* q, int64_t q_ld, const int64_t* q_index, const 
                      int64_t max_used, int64_t HQ, int64_t HK, int64_t D, float scale, int causal,
                      void* out_bf16, int64_t o_ld, float* lse, int64_t lse_ld, const int* work,
                      int64_t n_work, int v_bf16, hipStream_t stream);
+
+/*
+ * qx_attention_lse with work built for tile_rows query rows per workgroup
+ * (qx_paged_attention_tile_rows; 0: the default height). The rows' results
+ * are the same under either height, bit for bit.
+ */
+int qx_attention_lse_tiled(const void* q, int64_t q_ld, const int64_t* q_index, const void* k,
+                           const void* v, const int* cu_q, const int* used, const int* table,
+                           int64_t table_ld, const int* cu_k, int64_t seqs, int64_t max_q,
+                           int64_t max_used, int64_t HQ, int64_t HK, int64_t D, float scale,
+                           int causal, void* out_bf16, int64_t o_ld, float* lse, int64_t lse_ld,
+                           const int* work, int64_t n_work, int64_t tile_rows, int v_bf16,
+                           hipStream_t stream);
 
 /*
  * Replaces Engine.merge_attn_quant / the merge_attn_quant Triton kernel

@@ -60,6 +60,9 @@ SIGNATURES = {
     "qx_paged_attention_work": [_p, _p, _i64, _i64, _i64, _i64, _i32, _i64, _p, _i64],
     "qx_attention_lse": [_p, _i64, _p, _p, _p, _p, _p, _p, _i64, _p, _i64, _i64, _i64, _i64,
                          _i64, _i64, _f32, _i32, _p, _i64, _p, _i64, _p, _i64, _i32, _p],
+    "qx_attention_lse_tiled": [_p, _i64, _p, _p, _p, _p, _p, _p, _i64, _p, _i64, _i64, _i64,
+                               _i64, _i64, _i64, _f32, _i32, _p, _i64, _p, _i64, _p, _i64, _i64,
+                               _i32, _p],
     "qx_merge_attn_quant": [_p, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _i64, _i64, _p,
                             _i64, _p, _i64, _p],
     "qx_merge_partial": [_p, _i64, _p, _i64, _p, _p, _i64, _p, _i64, _i64, _i64, _i64, _p],

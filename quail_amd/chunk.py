@@ -462,7 +462,8 @@ def _pack_tree(arena, groups, *, timing=None, attention_heads=None):
     if attention_heads is not None:
         for tables in (segments, reads, reads and reads.get("nodes")):
             if tables:
-                tables["work"], tables["n_work"], _ = _work_list(tables, attention_heads)
+                tables["work"], tables["n_work"], tables["work_rows"] = _work_list(
+                    tables, attention_heads, choose_rows=True)
     ids = _cat(id_parts)
     positions = _cat(pos_parts)
     final = _cat(finals)

@@ -966,11 +966,24 @@ inline bool attn_rows_ok(int64_t D, int64_t G, int64_t rows) {
   return rows == attn_default_rows(G) || (D == 128 && attn_heads_per_group(G) == 4 && rows == 32);
 }
 
-// The 32-row tile is chosen when a pack's 64-row work items read at most
-// this many 64-key tiles on average (measured crossover on MI355X: 768-token
-// documents, 7.5 tiles per item, run 1.5% faster with it, 1024-token ones,
-// 9.5 tiles, 1.2% slower).
+// The 32-row tile is chosen (both sides measured on one MI355X, 32 heads, 8 KV
+// heads, times of 32 over 64 rows)
+//   - when the 64-row work items read at most this many 64-key tiles on
+//     average, where two workgroups a CU hide each other's fixed cost: 0.88 on
+//     128-token documents, 0.97 at 512 and 768 tokens; 1.00 at 4096, 1.02 at
+//     8000;
 constexpr double kShortItemTiles = 8.0;
+//   - when the 32-row items together read less than this many times the tiles
+//     of the 64-row ones (2 where every 64-row item is full): the second half
+//     of a 64-row workgroup whose sequence has few rows left works on nothing.
+//     20 documents of ~900 tokens, three 21-row questions on each: 56 us
+//     against 88; 64 of ~300, four 8-row questions: 80 against 155; 48-row
+//     questions (ratio 2): equal;
+constexpr double kHalfEmptyTiles = 1.7;
+//   - when the 64-row workgroups do not outnumber the CUs: the 32-row ones
+//     then spread one sequence over twice as many. One document of 700
+//     tokens 22.3 us against 29.7, of 2000 tokens 58.7 against 68.8.
+constexpr int64_t kCus = 256;
 
 }  // namespace
 }  // namespace qx
@@ -1088,18 +1101,32 @@ int qx_paged_attention_qnorm(const void* q, int64_t q_ld, const void* k_pool, co
 // of sequence s is row cu_k[s] + j of k (bf16) and v, rows of HK * D
 // elements. q_index (may be NULL): query row i reads Q row q_index[i].
 // v_bf16: V (pool or rows) holds bf16, else fp16.
+// tile_rows: the query rows per workgroup that `work` was built for.
+int qx_attention_lse_tiled(const void* q, int64_t q_ld, const int64_t* q_index, const void* k,
+                           const void* v, const int* cu_q, const int* used, const int* table,
+                           int64_t table_ld, const int* cu_k, int64_t seqs, int64_t max_q,
+                           int64_t max_used, int64_t HQ, int64_t HK, int64_t D, float scale,
+                           int causal, void* out_bf16, int64_t o_ld, float* lse, int64_t lse_ld,
+                           const int* work, int64_t n_work, int64_t tile_rows, int v_bf16,
+                           hipStream_t stream) {
+  QX_CHECK(out_bf16 && lse, "attention_lse: null output");
+  QX_CHECK((table == nullptr) != (cu_k == nullptr), "attention_lse: give a table or cu_k");
+  return qx::attention_impl(q, q_ld, q_index, k, v, cu_q, used, table, table_ld, cu_k, seqs,
+                            max_q, max_used, HQ, HK, D, qx::kPage, scale, causal, out_bf16,
+                            nullptr, o_ld, nullptr, 0, lse, lse_ld, work, n_work, tile_rows,
+                            v_bf16, stream);
+}
+
+// The same at the default tile height.
 int qx_attention_lse(const void* q, int64_t q_ld, const int64_t* q_index, const void* k,
                      const void* v, const int* cu_q, const int* used, const int* table,
                      int64_t table_ld, const int* cu_k, int64_t seqs, int64_t max_q,
                      int64_t max_used, int64_t HQ, int64_t HK, int64_t D, float scale, int causal,
                      void* out_bf16, int64_t o_ld, float* lse, int64_t lse_ld, const int* work,
                      int64_t n_work, int v_bf16, hipStream_t stream) {
-  QX_CHECK(out_bf16 && lse, "attention_lse: null output");
-  QX_CHECK((table == nullptr) != (cu_k == nullptr), "attention_lse: give a table or cu_k");
-  return qx::attention_impl(q, q_ld, q_index, k, v, cu_q, used, table, table_ld, cu_k, seqs,
-                            max_q, max_used, HQ, HK, D, qx::kPage, scale, causal, out_bf16,
-                            nullptr, o_ld, nullptr, 0, lse, lse_ld, work, n_work, 0, v_bf16,
-                            stream);
+  return qx_attention_lse_tiled(q, q_ld, q_index, k, v, cu_q, used, table, table_ld, cu_k, seqs,
+                                max_q, max_used, HQ, HK, D, scale, causal, out_bf16, o_ld, lse,
+                                lse_ld, work, n_work, 0, v_bf16, stream);
 }
 
 // The tree path's LSE merge fused with the o_proj input quantization
@@ -1153,8 +1180,8 @@ int qx_merge_partial(void* out, int64_t o_ld, float* lse, int64_t lse_ld, const 
 
 // Host function: the query rows per workgroup a paged call over these
 // sequences runs best with (the tile height to build its work list and call
-// it with): 32 where the configuration allows it and the 64-row work items
-// read at most kShortItemTiles 64-key tiles on average, else the default.
+// it with): 32 where the configuration allows it and one of the rules above
+// (kShortItemTiles, kHalfEmptyTiles, kCus) holds, else the default.
 int64_t qx_paged_attention_tile_rows(const int* cu_q, const int* used, int64_t seqs, int64_t HQ,
                                      int64_t HK, int64_t D, int causal) {
   if (!(cu_q && used && seqs >= 0 && HQ > 0 && HK > 0 && HQ % HK == 0)) {
@@ -1164,18 +1191,24 @@ int64_t qx_paged_attention_tile_rows(const int* cu_q, const int* used, int64_t s
   const int64_t G = HQ / HK;
   const int bq = qx::attn_default_rows(G);
   if (!qx::attn_rows_ok(D, G, 32) || bq == 32) return bq;
-  int64_t items = 0, tiles = 0;
+  int64_t items = 0, tiles = 0, tiles32 = 0;
   for (int64_t s = 0; s < seqs; ++s) {
     const int q_len = cu_q[s + 1] - cu_q[s];
     const int u = used[s];
-    for (int qt = 0; qt * bq < q_len; ++qt) {
-      const int last = std::min(qt * bq + bq, q_len) - 1;
-      const int keys = causal ? std::min(u, u - q_len + last + 1) : u;
-      tiles += (std::max(keys, 0) + 63) / 64;
-      ++items;
-    }
+    // 64-key tiles of the rows [first, first + rows) of the sequence
+    auto key_tiles = [&](int64_t first, int64_t rows) -> int64_t {
+      const int64_t last = std::min<int64_t>(first + rows, q_len) - 1;
+      const int64_t keys = causal ? std::min<int64_t>(u, u - q_len + last + 1) : u;
+      return (std::max<int64_t>(keys, 0) + 63) / 64;
+    };
+    for (int64_t r = 0; r < q_len; r += bq, ++items) tiles += key_tiles(r, bq);
+    for (int64_t r = 0; r < q_len; r += 32) tiles32 += key_tiles(r, 32);
   }
-  return items && (double)tiles <= qx::kShortItemTiles * (double)items ? 32 : bq;
+  const int64_t zgroups = HK * (G / qx::attn_heads_per_group(G));
+  const bool small = (double)tiles <= qx::kShortItemTiles * (double)items ||
+                     (double)tiles32 <= qx::kHalfEmptyTiles * (double)tiles ||
+                     items * zgroups <= qx::kCus;
+  return items && small ? 32 : bq;
 }
 
 // Host function: the work list of a paged call, one (sequence, query tile)

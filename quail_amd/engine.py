@@ -668,12 +668,14 @@ class Engine:
             work = None
         n_work = int(tables.get("n_work", 0)) if work is not None else 0
         seqs = tables["used"].shape[0]
-        _lib.call("qx_attention_lse", _ptr(q3), q3.stride(0), _ptr(q_index), _ptr(k), _ptr(v),
+        rows = int(tables.get("work_rows", 0)) if work is not None else 0
+        _lib.call("qx_attention_lse_tiled", _ptr(q3), q3.stride(0), _ptr(q_index), _ptr(k), _ptr(v),
                   _ptr(tables["cu_q"]), _ptr(tables["used"]), _ptr(table),
                   table.stride(0) if table is not None else 0, _ptr(cu_k), seqs,
                   int(tables["max_q"]), int(tables["max_used"]), hq, hk, d, scale,
                   int(tables.get("causal", True)), _ptr(out), out.stride(0), _ptr(lse),
-                  lse.stride(0), _ptr(work), n_work, int(v.dtype == torch.bfloat16), _stream())
+                  lse.stride(0), _ptr(work), n_work, rows, int(v.dtype == torch.bfloat16),
+                  _stream())
 
     def attention_unified(self, q3, k3, v3, meta, *, softmax_scale=None, output=None):
         """Write the chunk's KV to its pages, then one paged causal call with

@@ -92,6 +92,43 @@ def test_segments_call_matches_float32(hq, hk, d, v_dtype):
         torch.testing.assert_close(lse[:, r0:r1], l, atol=1e-3, rtol=0)
 
 
+@pytest.mark.parametrize("v_dtype", [torch.bfloat16, torch.float16])
+def test_lse_calls_at_both_tile_heights_are_bit_identical(v_dtype):
+    """Outputs and log-sum-exps of call A (causal, contiguous rows) and of
+    call B's form (not causal) are the same bits from 32-row workgroups, the
+    height that packs of short segments take, as from 64-row ones."""
+    from quail_amd.chunk import _work_list
+
+    hq, hk, d = 32, 8, 128
+    g = torch.Generator(device=DEV).manual_seed(5)
+    lengths = [5, 0, 64, 1, 300, 129, 33, 449]
+    cu = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    n = int(cu[-1])
+    q = torch.randn(n, hq * d, generator=g, device=DEV).to(torch.bfloat16)
+    k = torch.randn(n, hk * d, generator=g, device=DEV).to(torch.bfloat16)
+    v = torch.randn(n, hk * d, generator=g, device=DEV).to(v_dtype)
+    used = np.asarray(lengths, dtype=np.int32)
+    cu_t, used_t = torch.tensor(cu, device=DEV), torch.tensor(used, device=DEV)
+    for causal in (1, 0):
+        outs = []
+        for choose in (False, True):
+            work, n_work, rows = _work_list(dict(cu_q=cu, used=used, causal=causal), (hq, hk, d),
+                                            choose_rows=choose)
+            assert rows == (32 if choose else 0)
+            work = torch.tensor(work, device=DEV)
+            out = torch.full((n, hq * d), float("nan"), dtype=torch.bfloat16, device=DEV)
+            lse = torch.full((hq, n), float("nan"), dtype=torch.float32, device=DEV)
+            _lib.call("qx_attention_lse_tiled", _p(q), q.stride(0), None, _p(k), _p(v), _p(cu_t),
+                      _p(used_t), None, 0, _p(cu_t), len(lengths), max(lengths), max(lengths),
+                      hq, hk, d, float(d ** -0.5), causal, _p(out), out.stride(0), _p(lse),
+                      lse.stride(0), _p(work), n_work, rows, int(v_dtype == torch.bfloat16),
+                      _stream())
+            torch.cuda.synchronize()
+            outs.append((out, lse))
+        assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+        assert bool(torch.isfinite(outs[0][1]).all())
+
+
 def test_page_reads_with_row_index_match_float32():
     """Call B: selected query rows (q_index), not causal, keys through block
     tables over 16-row pages (used not a page multiple)."""

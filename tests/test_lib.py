@@ -93,6 +93,27 @@ def test_attention_tile_rows_choice_and_32_row_work_list():
                    128, 1, 32, work.ctypes.data, 32)
 
 
+def test_attention_tile_rows_for_half_empty_and_few_workgroups():
+    """32 query rows per workgroup also for sequences that leave the second
+    half of a 64-row workgroup empty (few rows over many keys) and for calls
+    whose 64-row workgroups do not outnumber the 256 CUs; 64 where 64-row
+    workgroups are full, long and many."""
+    import numpy as np
+
+    def rows(q_lens, used, causal=1):
+        cu_q = np.concatenate([[0], np.cumsum(q_lens)]).astype(np.int32)
+        used = np.asarray(used, dtype=np.int32)
+        return _lib.count("qx_paged_attention_tile_rows", cu_q.ctypes.data, used.ctypes.data,
+                          len(used), 32, 8, 128, causal)
+
+    assert rows([21] * 60, [921] * 60) == 32
+    assert rows([21] * 60, [900] * 60, causal=0) == 32
+    assert rows([48] * 240, [2048] * 240) == 64
+    assert rows([2000], [2000]) == 32       # 32 items x 8 head groups = 256 workgroups
+    assert rows([2112], [2112]) == 64
+    assert rows([], []) == 64
+
+
 def test_gemm_config_choice_by_shape(monkeypatch):
     """The arithmetic family is a function of N alone: widths that are a
     multiple of 256 or 320 take the promotion family (config 31's 256 x 320
