@@ -22,6 +22,38 @@ namespace {
 
 constexpr int kRowThreads = 256;  // 4 rows (one per wave) per workgroup
 
+// One 8-column chunk of a normed row: y from the row's values, the weight's
+// 16 bytes and rstd, at the rounding points of each MODE.
+template <int MODE>
+__device__ __forceinline__ void norm_row_chunk(const float (&v)[8], const uint4& wv, float rstd,
+                                               float (&y)[8]) {
+  const uint32_t ww[4] = {wv.x, wv.y, wv.z, wv.w};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float w0 = lo_bf16(ww[k]), w1 = hi_bf16(ww[k]);
+    if (MODE == 0) {
+      y[2 * k] = v[2 * k] * rstd * w0;
+      y[2 * k + 1] = v[2 * k + 1] * rstd * w1;
+    } else {
+      y[2 * k] = round_bf16(round_bf16(v[2 * k] * rstd) * w0);
+      y[2 * k + 1] = round_bf16(round_bf16(v[2 * k + 1] * rstd) * w1);
+    }
+  }
+}
+
+// The chunk's e4m3 bytes under its group's scale, which one lane stores.
+__device__ __forceinline__ void quant_chunk(const float (&y)[8], float scale, uint8_t* out,
+                                            bool first, float* scale_out) {
+  const float rs = recip(scale);
+  uint2 o;
+  o.x = pack4_fp8(div_by(y[0], scale, rs), div_by(y[1], scale, rs), div_by(y[2], scale, rs),
+                  div_by(y[3], scale, rs));
+  o.y = pack4_fp8(div_by(y[4], scale, rs), div_by(y[5], scale, rs), div_by(y[6], scale, rs),
+                  div_by(y[7], scale, rs));
+  *reinterpret_cast<uint2*>(out) = o;
+  if (first) *scale_out = scale;
+}
+
 // ---------------------------------------------------------------------------
 // Row norm + quant. One wave per token row; lane holds chunks of 8 columns
 // (16 B of bf16): chunk c = lane + 64 * i. A 128-column group is 16 chunks,
@@ -95,35 +127,117 @@ __global__ __launch_bounds__(kRowThreads) void norm_quant_kernel(
     float y[8];
     float amax = 0.f;
     if (live) {
-      uint4 wv = *reinterpret_cast<const uint4*>(w + c * 8);
-      uint32_t ww[4] = {wv.x, wv.y, wv.z, wv.w};
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        float w0 = lo_bf16(ww[k]), w1 = hi_bf16(ww[k]);
-        if (MODE == 0) {
-          y[2 * k] = v[i][2 * k] * rstd * w0;
-          y[2 * k + 1] = v[i][2 * k + 1] * rstd * w1;
-        } else {
-          y[2 * k] = round_bf16(round_bf16(v[i][2 * k] * rstd) * w0);
-          y[2 * k + 1] = round_bf16(round_bf16(v[i][2 * k + 1] * rstd) * w1);
-        }
-      }
+      norm_row_chunk<MODE>(v[i], *reinterpret_cast<const uint4*>(w + c * 8), rstd, y);
 #pragma unroll
       for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(y[k]));
     }
     amax = group_max<16>(amax);
-    const float scale = fp8_scale(amax);
-    const float rs = recip(scale);
-    if (live) {
-      uint2 o;
-      o.x = pack4_fp8(div_by(y[0], scale, rs), div_by(y[1], scale, rs), div_by(y[2], scale, rs),
-                      div_by(y[3], scale, rs));
-      o.y = pack4_fp8(div_by(y[4], scale, rs), div_by(y[5], scale, rs), div_by(y[6], scale, rs),
-                      div_by(y[7], scale, rs));
-      *reinterpret_cast<uint2*>(qrow + c * 8) = o;
-      if ((lane & 15) == 0) scales[(int64_t)(c >> 4) * s_ld + row] = scale;
+    if (live) quant_chunk(y, fp8_scale(amax), qrow + c * 8, (lane & 15) == 0,
+                          scales + (int64_t)(c >> 4) * s_ld + row);
+  }
+}
+
+// The same with one workgroup of WPR waves per row, each holding NITER / WPR
+// of the row's passes. Every lane's sum of squares runs over its chunks in
+// the one-wave kernel's order (through LDS), so a row's bits are the same.
+// For few rows the one-wave kernel is its own chain of instructions (load,
+// sum, then NITER passes of group maximum, division and packing in turn);
+// here the passes run side by side and the weights load with the row.
+template <int NITER, int WPR, int MODE>
+__global__ __launch_bounds__(64 * WPR) void norm_quant_row_kernel(
+    const uint16_t* __restrict__ x, int64_t x_ld, uint16_t* __restrict__ res, int64_t res_ld,
+    const int64_t* __restrict__ ids, const uint16_t* __restrict__ w, uint8_t* __restrict__ q,
+    int64_t q_ld, float* __restrict__ scales, int64_t s_ld, int H, float eps) {
+  constexpr int PER = (NITER + WPR - 1) / WPR;
+  __shared__ float4 vals[NITER][2][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row = blockIdx.x;
+  const int nch = H >> 3;
+  const uint16_t* xrow = x + (MODE == 2 ? ids[row] : (int64_t)row) * x_ld;
+  uint16_t* rrow = MODE == 1 ? nullptr : res + (int64_t)row * res_ld;
+  uint4 a[PER], r[PER], wv[PER];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int c = lane + 64 * (wave + j * WPR);
+    if (c < nch) {
+      a[j] = *reinterpret_cast<const uint4*>(xrow + c * 8);
+      if (MODE == 0) r[j] = *reinterpret_cast<const uint4*>(rrow + c * 8);
+      wv[j] = *reinterpret_cast<const uint4*>(w + c * 8);
     }
   }
+  float v[PER][8];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int i = wave + j * WPR;
+    const int c = lane + 64 * i;
+    if (c >= nch) continue;
+    const uint32_t aw[4] = {a[j].x, a[j].y, a[j].z, a[j].w};
+    if (MODE == 0) {
+      const uint32_t rw[4] = {r[j].x, r[j].y, r[j].z, r[j].w};
+      uint32_t o[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        v[j][2 * k] = lo_bf16(aw[k]) + lo_bf16(rw[k]);
+        v[j][2 * k + 1] = hi_bf16(aw[k]) + hi_bf16(rw[k]);
+        o[k] = pack2_bf16(v[j][2 * k], v[j][2 * k + 1]);
+      }
+      *reinterpret_cast<uint4*>(rrow + c * 8) = make_uint4(o[0], o[1], o[2], o[3]);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        v[j][2 * k] = lo_bf16(aw[k]);
+        v[j][2 * k + 1] = hi_bf16(aw[k]);
+      }
+      if (MODE == 2) *reinterpret_cast<uint4*>(rrow + c * 8) = a[j];
+    }
+    vals[i][0][lane] = make_float4(v[j][0], v[j][1], v[j][2], v[j][3]);
+    vals[i][1][lane] = make_float4(v[j][4], v[j][5], v[j][6], v[j][7]);
+  }
+  __syncthreads();
+  float ss = 0.f;
+#pragma unroll
+  for (int i = 0; i < NITER; ++i) {
+    if (lane + 64 * i < nch) {
+      const float4 lo = vals[i][0][lane], hi = vals[i][1][lane];
+      const float s[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+      for (int k = 0; k < 8; ++k) ss += s[k] * s[k];
+    }
+  }
+  ss = group_sum<64>(ss);
+  const float rstd = 1.0f / sqrtf(ss / (float)H + eps);
+  uint8_t* qrow = q + (int64_t)row * q_ld;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int c = lane + 64 * (wave + j * WPR);
+    if (64 * (wave + j * WPR) >= nch) break;  // wave-uniform
+    const bool live = c < nch;
+    float y[8];
+    float amax = 0.f;
+    if (live) {
+      norm_row_chunk<MODE>(v[j], wv[j], rstd, y);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(y[k]));
+    }
+    amax = group_max<16>(amax);
+    if (live) quant_chunk(y, fp8_scale(amax), qrow + c * 8, (lane & 15) == 0,
+                          scales + (int64_t)(c >> 4) * s_ld + row);
+  }
+}
+
+// Whether a row gets a workgroup of its own (norm_quant_row_kernel) or a wave.
+// Measured (us, a wave -> a workgroup per row): MODE 0, hidden 2560: 333 rows
+// 5.9 -> 3.9, 1003 6.7 -> 5.2, 2048 8.1 -> 8.4, 4096 14.4 -> 14.2, 16384 47.0
+// -> 45.9; hidden 5120: 333 9.8 -> 5.3, 2048 16.9 -> 14.2, 16384 126.9 ->
+// 103.0; MODE 1, hidden 2560: 333 5.2 -> 3.9, 2048 6.5 -> 7.8, 16384 27.1 ->
+// 35.5; hidden 5120: 16384 54.7 -> 59.4; hidden 8192: 16384 134 -> 112; MODE
+// 2, hidden 2560: 333 5.6 -> 4.1, 4096 12.6 -> 13.6; hidden 5120: 16384 106.5
+// -> 86.5; hidden 128: 2.8 -> 2.9 at any few rows.
+bool row_workgroups(int niter, int mode, int n) {
+  if (niter < 2) return false;
+  if (n <= 1536 || niter > (mode == 1 ? 10 : 8)) return true;
+  return mode == 0 && niter >= 5 && n >= 4096;
 }
 
 template <int MODE>
@@ -133,11 +247,19 @@ int launch_norm_quant(const void* x, int64_t x_ld, void* res, int64_t res_ld, co
   const int niter = (H / 8 + 63) / 64;
   dim3 grid((n + 3) / 4), block(kRowThreads);
 #define QX_NQ_CASE(NI)                                                                     \
-  case NI:                                                                                 \
-    hipLaunchKernelGGL((norm_quant_kernel<NI, MODE>), grid, block, 0, stream,              \
-                       (const uint16_t*)x, x_ld, (uint16_t*)res, res_ld, ids,              \
-                       (const uint16_t*)w, (uint8_t*)q, q_ld, scales, s_ld, n, H, eps);    \
-    break;
+  case NI: {                                                                               \
+    constexpr int kWaves = NI <= 8 ? NI : (NI + 1) / 2;                                    \
+    if (row_workgroups(NI, MODE, n))                                                       \
+      hipLaunchKernelGGL((norm_quant_row_kernel<NI, kWaves, MODE>), dim3(n),               \
+                         dim3(64 * kWaves), 0, stream, (const uint16_t*)x, x_ld,           \
+                         (uint16_t*)res, res_ld, ids, (const uint16_t*)w, (uint8_t*)q,     \
+                         q_ld, scales, s_ld, H, eps);                                      \
+    else                                                                                   \
+      hipLaunchKernelGGL((norm_quant_kernel<NI, MODE>), grid, block, 0, stream,            \
+                         (const uint16_t*)x, x_ld, (uint16_t*)res, res_ld, ids,            \
+                         (const uint16_t*)w, (uint8_t*)q, q_ld, scales, s_ld, n, H, eps);  \
+    break;                                                                                 \
+  }
   switch (niter) {
     QX_NQ_CASE(1)
     QX_NQ_CASE(2)

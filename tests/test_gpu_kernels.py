@@ -429,6 +429,34 @@ def test_add_rmsnorm_quant(n, h):
     _fp8_close(q, s, q_ref, s_ref)
 
 
+@pytest.mark.parametrize("h", [384, 640, 2560, 4096, 5120, 8192])
+def test_norm_quant_rows_do_not_depend_on_how_many_share_the_launch(h):
+    """Rows of launches whose rows have a wave each (1537 rows; 2048 to 4095
+    with a residual) are the same bits as alone, where a row has a workgroup
+    of its own, in all three forms."""
+    g = _gen(h)
+    eng = _engine(4, 2, 64)
+    n = 1537
+    x = torch.randn(n, h, generator=g).to(torch.bfloat16).to(DEV)
+    r = torch.randn(n, h, generator=g).to(torch.bfloat16).to(DEV)
+    norm = type("N", (), {"weight": (1 + 0.1 * torch.randn(h, generator=g)).to(
+        torch.bfloat16).to(DEV), "variance_epsilon": 1e-6})()
+    ids = torch.randint(0, n, (n,), generator=g).to(DEV)
+
+    def forms(rows):
+        res = r[rows].clone()
+        q0, s0 = eng.norm_quant(x[rows], norm, res)
+        q1, s1 = eng.norm_quant(x[rows], norm)
+        q2, s2, e = eng.embed_norm_quant(ids[rows], x, norm)
+        return [q0.view(torch.uint8), s0, res, q1.view(torch.uint8), s1, q2.view(torch.uint8),
+                s2, e]
+
+    whole = forms(slice(0, n))
+    for rows in (slice(0, 1), slice(700, 737), slice(n - 1, n), slice(1, n)):
+        for a, b in zip(forms(rows), whole):
+            assert torch.equal(a, b[rows])
+
+
 @pytest.mark.parametrize("n,h", [(3, 256), (64, 2560)])
 def test_rmsnorm_quant_and_embed_fused(n, h):
     g = _gen(7 * n + h)
