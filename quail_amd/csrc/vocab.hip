@@ -43,8 +43,6 @@ __device__ __forceinline__ float bf16_round(float v) {
   return static_cast<float>(static_cast<__bf16>(v));
 }
 
-constexpr int kStages = 3;
-
 // 128-byte LDS rows of 8 16-byte chunks, chunk-swizzled by (row >> 1) & 7:
 // the 16 rows one quarter-wave's ds_read_b128 touches then cover all banks
 __device__ __forceinline__ int vswz(int row) { return (row >> 1) & 7; }
@@ -68,11 +66,19 @@ __device__ __forceinline__ void load_slab(const uint16_t* __restrict__ g, int64_
 }
 
 // A workgroup of 4 waves covers 128 head rows (32 per wave) and TM 32-token
-// tiles; 64 K elements per stage (head 16 KiB + tokens 4 KiB per tile),
-// three stages. The MFMA fragment of k-step s for lane half hh is K
+// tiles; 64 K elements per stage (head 16 KiB + tokens 4 KiB per tile). A
+// workgroup starts at its own K chunk and wraps around: at a hidden size of
+// 4096 the head's rows are 8 KiB apart, and workgroups that all read the same
+// columns of their rows kept to a part of the memory channels (37 tokens,
+// V = 151936: 259 -> 218 us, 4.8 -> 5.7 TB/s; at 2560 and 5120, whose rows
+// spread over the channels by themselves, no change). Three stages; two, and
+// so two workgroups a CU at TM = 4, where several token blocks share each
+// head block and the launch waits for the L2 and the matrix cores more than
+// for memory (300 tokens: 833 -> 704 us; 128 tokens, one block, at hidden
+// 2560: three stages 203 us, two 214). The MFMA fragment of k-step s for lane half hh is K
 // elements [32 hh + 8 s, +8) of the chunk (16-byte chunk 4 hh + s), the
 // same permutation for both operands.
-template <int TM>
+template <int TM, int kStages>
 __global__ __launch_bounds__(256) void vocab_lse_kernel(
     const uint16_t* __restrict__ x, int64_t x_ld, const uint16_t* __restrict__ head,
     int64_t h_ld, const int64_t* __restrict__ targets, int t, float2* __restrict__ part,
@@ -93,7 +99,9 @@ __global__ __launch_bounds__(256) void vocab_lse_kernel(
   const int tok0 = blockIdx.y * (32 * TM);
   const int KC = H >> 6;
 
-  auto issue = [&](int kc, int stage) {
+  const int rotate = (int)(blockIdx.x % KC);
+  auto issue = [&](int step, int stage) {
+    const int kc = step + rotate < KC ? step + rotate : step + rotate - KC;
     uint8_t* buf = smem + stage * kStage;
 #pragma unroll
     for (int j = 0; j < kSlabsPerWave; ++j) {
@@ -114,8 +122,8 @@ __global__ __launch_bounds__(256) void vocab_lse_kernel(
     if (st < KC) issue(st, st);
   for (int kc = 0; kc < KC; ++kc) {
     const int stage = kc % kStages;
-    if (kc + 1 < KC) {
-      wait_vmcnt<kSlabsPerWave>();  // chunk kc landed; kc + 1 may be in flight
+    if (kc + kStages - 1 <= KC) {
+      wait_vmcnt<(kStages - 2) * kSlabsPerWave>();  // chunk kc landed; later ones may be in flight
     } else {
       wait_vmcnt<0>();
     }
@@ -190,23 +198,48 @@ __global__ __launch_bounds__(256) void vocab_lse_kernel(
   }
 }
 
-__global__ __launch_bounds__(64) void vocab_finish_kernel(const float2* __restrict__ part,
-                                                          int nblk, const float* __restrict__ tlogit,
-                                                          int t, float* __restrict__ out,
-                                                          int64_t out_ld, int n) {
+// One workgroup per token. A thread's partials are loaded before any is
+// merged: their addresses are known at once, and merging each as it came
+// made every one of one wave's 19 loads a memory round trip of its own (37
+// tokens at Qwen3's vocabulary: 14.0 -> 5.6 us).
+constexpr int kFinishThreads = 512;
+
+__global__ __launch_bounds__(kFinishThreads) void vocab_finish_kernel(
+    const float2* __restrict__ part, int nblk, const float* __restrict__ tlogit, int t,
+    float* __restrict__ out, int64_t out_ld, int n) {
+  constexpr int kAhead = 4;
+  constexpr int kFinishWaves = kFinishThreads / 64;
+  __shared__ float2 red[kFinishWaves];
   const int tok = blockIdx.x;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  float target = 0.0f;
+  if ((int)threadIdx.x < t) target = tlogit[(int64_t)tok * t + threadIdx.x];
   float2 acc = make_float2(-INFINITY, 0.0f);
-  for (int b = lane; b < nblk; b += 64) acc = lse_merge(acc, part[(int64_t)b * n + tok]);
+  for (int b0 = threadIdx.x; b0 < nblk; b0 += kAhead * kFinishThreads) {
+    float2 p[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int b = b0 + u * kFinishThreads;
+      p[u] = b < nblk ? part[(int64_t)b * n + tok] : make_float2(-INFINITY, 0.0f);
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) acc = lse_merge(acc, p[u]);
+  }
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) {
     const float2 o = make_float2(__shfl_xor(acc.x, off), __shfl_xor(acc.y, off));
     acc = lse_merge(acc, o);
   }
   // the butterfly leaves each lane a sum in its own association order, which
-  // may differ in the last bit: every target takes lane 0's
-  const float lse = __shfl(acc.x + __log2f(acc.y) * kLn2, 0);
-  if (lane < t) out[(int64_t)tok * out_ld + lane] = tlogit[(int64_t)tok * t + lane] - lse;
+  // may differ in the last bit: lane 0's is the wave's
+  if (lane == 0) red[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if ((int)threadIdx.x < t) {
+    float2 all = red[0];
+#pragma unroll
+    for (int w = 1; w < kFinishWaves; ++w) all = lse_merge(all, red[w]);
+    out[(int64_t)tok * out_ld + threadIdx.x] = target - (all.x + __log2f(all.y) * kLn2);
+  }
 }
 
 // head rows per workgroup
@@ -250,22 +283,25 @@ int vocab_run(const void* normed, int64_t n_ld, const void* head, int64_t h_ld,
   const dim3 grid(nblk, (unsigned)((n + 32 * tm - 1) / (32 * tm)));
   const auto* xp = reinterpret_cast<const uint16_t*>(normed);
   const auto* hp = reinterpret_cast<const uint16_t*>(head);
+#define QX_VOCAB(TM, STAGES)                                                                  \
+  hipLaunchKernelGGL((vocab_lse_kernel<TM, STAGES>), grid, dim3(256), 0, stream, xp, n_ld, hp, \
+                     h_ld, targets, (int)t, part, tlogit, (int)n, (int)V, (int)H)
   if (tm == 1) {
-    hipLaunchKernelGGL(vocab_lse_kernel<1>, grid, dim3(256), 0, stream, xp, n_ld, hp, h_ld,
-                       targets, (int)t, part, tlogit, (int)n, (int)V, (int)H);
+    QX_VOCAB(1, 3);
   } else if (tm == 2) {
-    hipLaunchKernelGGL(vocab_lse_kernel<2>, grid, dim3(256), 0, stream, xp, n_ld, hp, h_ld,
-                       targets, (int)t, part, tlogit, (int)n, (int)V, (int)H);
+    QX_VOCAB(2, 3);
+  } else if (grid.y == 1) {
+    QX_VOCAB(4, 3);
   } else {
-    hipLaunchKernelGGL(vocab_lse_kernel<4>, grid, dim3(256), 0, stream, xp, n_ld, hp, h_ld,
-                       targets, (int)t, part, tlogit, (int)n, (int)V, (int)H);
+    QX_VOCAB(4, 2);
   }
+#undef QX_VOCAB
   {
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
   }
-  hipLaunchKernelGGL(vocab_finish_kernel, dim3((unsigned)n), dim3(64), 0, stream, part, nblk,
-                     tlogit, (int)t, out, out_ld, (int)n);
+  hipLaunchKernelGGL(vocab_finish_kernel, dim3((unsigned)n), dim3(kFinishThreads), 0,
+                     stream, part, nblk, tlogit, (int)t, out, out_ld, (int)n);
   QX_LAUNCH_STATUS();
 }
 
