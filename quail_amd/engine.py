@@ -53,12 +53,26 @@ GEMM_ODD_WIDTH_CONFIG = 11
 CUS = 256
 
 
+_environ = getattr(os.environ, "_data", None)   # the dict os.environ wraps
+
+
+def _forced(name):
+    """os.environ.get(name). Each GEMM asks; os.environ encodes the name and
+    raises and catches KeyError every time (1.6 us against 0.2)."""
+    if type(_environ) is not dict or os.name != "posix":
+        return os.environ.get(name)
+    value = _environ.get(name.encode())
+    return None if value is None else os.fsdecode(value)
+
+
 def _ptr(t):
     return None if t is None else t.data_ptr()
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    """The handle of the current stream of the current device (without the
+    Stream object torch.cuda.current_stream() makes around it)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def gemm_config(n: int, k: int, m: int) -> int:
@@ -67,8 +81,10 @@ def gemm_config(n: int, k: int, m: int) -> int:
     where they take fewer full-wave units, or where 256 x 256 ones cannot
     tile N), config 11 for the rest."""
     forced = os.environ.get(GEMM_CONFIG_ENV)
-    if forced is not None:
-        return int(forced)
+    return _family_config(n, m) if forced is None else int(forced)
+
+
+def _family_config(n: int, m: int) -> int:
     if n % 256 == 0 or n % 320 == 0:
         if n % 320 == 0 and (n % 256 or _wide_tiles_fill_better(n, m)):
             return GEMM_PROMOTION_WIDE_CONFIG
@@ -135,10 +151,15 @@ def _fastest_tile(n: int, k: int, m: int, swiglu: bool, large: int) -> int:
 def gemm_tiles(n: int, k: int, m: int) -> int:
     """The config Engine.gemm launches: gemm_config's, and within the
     promotion family the tile that takes least time at m rows."""
-    config = gemm_config(n, k, m)
-    if config not in PROMOTION_CONFIGS or GEMM_CONFIG_ENV in os.environ:
-        return config
-    return _fastest_tile(n, k, m, False, config)
+    if _forced(GEMM_CONFIG_ENV) is not None:
+        return gemm_config(n, k, m)
+    return _tiles(n, k, m)
+
+
+@functools.lru_cache(maxsize=4096)
+def _tiles(n: int, k: int, m: int) -> int:
+    config = _family_config(n, m)
+    return _fastest_tile(n, k, m, False, config) if config in PROMOTION_CONFIGS else config
 
 
 SWIGLU_CONFIG_ENV = "QUAIL_SWIGLU_CONFIG"
@@ -151,7 +172,7 @@ def swiglu_config(n: int = 0, k: int = 0, m: int = 0) -> int:
     family) stay selectable. QUAIL_SWIGLU_CONFIG forces it alone,
     QUAIL_GEMM_CONFIG with every GEMM."""
     for env in (SWIGLU_CONFIG_ENV, GEMM_CONFIG_ENV):
-        forced = os.environ.get(env)
+        forced = _forced(env)
         if forced is not None and int(forced) in (10, 22, 30) + SWIGLU_SMALL_CONFIGS:
             return int(forced)
     return _fastest_tile(n, k, m, True, SWIGLU_DEFAULT_CONFIG)
@@ -209,8 +230,9 @@ class Engine:
         raise AttributeError(f"no weight scale on {type(linear).__name__}")
 
     def _col_major_scales(self, num_tokens, width, device="cuda"):
-        return torch.empty((width // GROUP, num_tokens), dtype=torch.float32,
-                           device=device).permute(1, 0)
+        # the (tokens, groups) view of (groups, tokens) storage, in one call
+        return torch.empty_strided((num_tokens, width // GROUP), (1, max(num_tokens, 1)),
+                                   dtype=torch.float32, device=device)
 
     @staticmethod
     def _scale_ld(scales):
