@@ -120,9 +120,9 @@ def _wide_tiles_fill_better(n: int, m: int) -> bool:
 # 7% at most, against the fastest tile of each of those 348 launches.
 PROMOTION_TILES = {
     40: (16, 32, 256, 0.167, 2.9), 41: (32, 32, 512, 0.220, 3.4),
-    42: (64, 64, 256, 0.302, 3.8), 43: (128, 64, 256, 0.442, 4.3),
-    44: (192, 64, 256, 0.539, 4.6), 45: (128, 128, 256, 0.602, 6.3),
-    46: (192, 128, 256, 0.781, 7.0), 47: (256, 128, 256, 0.979, 7.9),
+    42: (64, 64, 256, 0.296, 3.8), 43: (128, 64, 256, 0.419, 4.3),
+    44: (192, 64, 256, 0.539, 4.6), 45: (128, 128, 256, 0.560, 6.3),
+    46: (192, 128, 256, 0.750, 7.0), 47: (256, 128, 256, 0.979, 7.9),
     30: (256, 256, 256, 1.443, 3.9), 31: (256, 320, 256, 1.686, 10.0),
 }
 # the same with the SiLU-quant epilogue
