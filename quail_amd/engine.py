@@ -131,18 +131,23 @@ SWIGLU_TILES = {48: (64, 256, 256, 1.369, -4.0), 49: (96, 256, 256, 1.380, -0.5)
 SWIGLU_SMALL_CONFIGS = (48, 49, 50)
 
 
+def _tile_cost(tile, n: int, k: int, m: int) -> float:
+    """us of an (m x k) by (n x k) launch on `tile` (a row of the tables above)."""
+    bm, bn, at_once, block, rest = tile
+    rounds = -(-(-(-m // bm) * (n // bn)) // at_once)
+    return rounds * (rest + k // GROUP * block)
+
+
 @functools.lru_cache(maxsize=4096)
 def _fastest_tile(n: int, k: int, m: int, swiglu: bool, large: int) -> int:
     """The tile config of an (m x k) by (n x k) promotion GEMM: `large` (30
     or 31) unless a smaller tile's measured cost is below its. A row's bits
     are the same under all of them."""
     best, cost = large, None
-    for config, (bm, bn, at_once, block, rest) in (SWIGLU_TILES if swiglu
-                                                   else PROMOTION_TILES).items():
-        if n % bn or (config in PROMOTION_CONFIGS and config != large):
+    for config, tile in (SWIGLU_TILES if swiglu else PROMOTION_TILES).items():
+        if n % tile[1] or (config in PROMOTION_CONFIGS and config != large):
             continue
-        rounds = -(-(-(-m // bm) * (n // bn)) // at_once)
-        c = rounds * (rest + k // GROUP * block)
+        c = _tile_cost(tile, n, k, m)
         if cost is None or c < cost:
             best, cost = config, c
     return best
@@ -165,17 +170,50 @@ def _tiles(n: int, k: int, m: int) -> int:
 SWIGLU_CONFIG_ENV = "QUAIL_SWIGLU_CONFIG"
 
 
-def swiglu_config(n: int = 0, k: int = 0, m: int = 0) -> int:
-    """Tile schedule of the gate_up GEMM with the SiLU-quant epilogue (n =
-    gate_up rows, 256 per tile): the promotion form, on the tile that takes
-    least time at m rows (30's 256 x 256 for packs); 10 and 22 (the rescale
-    family) stay selectable. QUAIL_SWIGLU_CONFIG forces it alone,
-    QUAIL_GEMM_CONFIG with every GEMM."""
+def _forced_swiglu():
     for env in (SWIGLU_CONFIG_ENV, GEMM_CONFIG_ENV):
         forced = _forced(env)
         if forced is not None and int(forced) in (10, 22, 30) + SWIGLU_SMALL_CONFIGS:
             return int(forced)
-    return _fastest_tile(n, k, m, True, SWIGLU_DEFAULT_CONFIG)
+    return None
+
+
+def swiglu_config(n: int = 0, k: int = 0, m: int = 0) -> int:
+    """Tile schedule of one gate_up launch with the SiLU-quant epilogue (n =
+    gate_up rows, 256 per tile): the promotion form, on the tile that takes
+    least time at m rows (30's 256 x 256 for packs); 10 and 22 (the rescale
+    family) stay selectable. QUAIL_SWIGLU_CONFIG forces it alone,
+    QUAIL_GEMM_CONFIG with every GEMM."""
+    forced = _forced_swiglu()
+    return _fastest_tile(n, k, m, True, SWIGLU_DEFAULT_CONFIG) if forced is None else forced
+
+
+def swiglu_launches(n: int, k: int, m: int) -> tuple:
+    """The (rows, config) launches of a gate_up projection of m rows, first
+    rows first: one, or two as _swiglu_launches has it."""
+    forced = _forced_swiglu()
+    return _swiglu_launches(n, k, m) if forced is None else ((m, forced),)
+
+
+@functools.lru_cache(maxsize=4096)
+def _swiglu_launches(n: int, k: int, m: int) -> tuple:
+    """One launch on the fastest tile, or the whole 256-row tiles on config 30
+    and the rest on a small tile where the two by the table take less: a few
+    rows past a multiple of 256 otherwise cost a whole row of 256 x 256 tiles
+    and often another round of the CUs. Measured (us, best one launch / two):
+    Qwen3-4B 800 rows 75 / 59, 1003 77 / 66; -8B 1300 rows 162 / 138; -32B 277
+    rows 142 / 129, 800 278 / 258; the table's choice was the faster one, or
+    within 4% of it, at each of 33 sizes from 256 to 1300 rows. The rest costs
+    less than the table says (the first launch leaves its weights in cache)."""
+    config = _fastest_tile(n, k, m, True, SWIGLU_DEFAULT_CONFIG)
+    first = m // 256 * 256
+    if 0 < first < m:
+        rest = _fastest_tile(n, k, m - first, True, SWIGLU_DEFAULT_CONFIG)
+        two = (_tile_cost(SWIGLU_TILES[30], n, k, first) +
+               _tile_cost(SWIGLU_TILES[rest], n, k, m - first))
+        if rest != 30 and two < _tile_cost(SWIGLU_TILES[config], n, k, m):
+            return ((first, 30), (m - first, rest))
+    return ((m, config),)
 
 
 class Engine:
@@ -295,10 +333,15 @@ class Engine:
         if timed:
             start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             start.record()
-        _lib.call("qx_gemm_fp8_swiglu_quant", _ptr(q_input), _ptr(input_scale), _ptr(w),
-                  _ptr(sw), _ptr(q), q.stride(0), _ptr(scales), self._scale_ld(scales), m, half,
-                  k, q_input.stride(0), self._scale_ld(input_scale), swiglu_config(n, k, m),
-                  _stream())
+        row = 0
+        for rows, config in swiglu_launches(n, k, m):
+            # e4m3 rows and column-major scales of the launch's first row
+            _lib.call("qx_gemm_fp8_swiglu_quant", _ptr(q_input) + row * q_input.stride(0),
+                      _ptr(input_scale) + 4 * row, _ptr(w), _ptr(sw),
+                      _ptr(q) + row * q.stride(0), q.stride(0), _ptr(scales) + 4 * row,
+                      self._scale_ld(scales), rows, half, k, q_input.stride(0),
+                      self._scale_ld(input_scale), config, _stream())
+            row += rows
         if timed:
             end.record()
             self.gemm_timer.append((m, n, k, start, end, True))

@@ -414,6 +414,34 @@ def test_gemm_rejects_bad_shapes():
 
 # ---- norms and quant ------------------------------------------------------------
 
+def test_gate_up_in_two_launches_is_bit_identical(monkeypatch):
+    """277 rows whose gate_up goes out as 256 rows on 256 x 256 tiles and 21 on
+    64 x 256 ones: the codes and scales of one launch, bit for bit, also from
+    rows inside a wider matrix."""
+    from quail_amd import engine
+
+    g = _gen(277)
+    m, n, k = 277, 51200, 2560
+    assert engine.swiglu_launches(n, k, m) == ((256, 30), (21, 48))
+    gd = torch.Generator(device=DEV).manual_seed(277)
+    w = torch.randint(0, 256, (n, k), generator=gd, device=DEV, dtype=torch.uint8)
+    w = torch.where((w & 127) == 127, w - 1, w)      # no NaN codes
+    sw = torch.rand(n // 128, k // 128, generator=gd, device=DEV) * 1e-3
+    lin = type("L", (), {"weight": w.view(torch.float8_e4m3fn), "weight_scale_inv": sw})()
+    eng = _engine(4, 2, 64)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16).to(DEV)
+    q, s = eng.quant(x)
+    wide = torch.empty(m, k + 256, dtype=torch.float8_e4m3fn, device=DEV)
+    wide[:, :k] = q
+    got = eng.gate_up_activation_quant(q, s, lin)
+    strided = eng.gate_up_activation_quant(wide[:, :k], s, lin)
+    monkeypatch.setenv(engine.SWIGLU_CONFIG_ENV, "30")
+    want = eng.gate_up_activation_quant(q, s, lin)
+    for a, b in ((got, want), (strided, want)):
+        assert torch.equal(a[0].view(torch.uint8), b[0].view(torch.uint8))
+        assert torch.equal(a[1], b[1])
+
+
 @pytest.mark.parametrize("n,h", [(1, 256), (37, 2560), (130, 5120), (5, 4096)])
 def test_add_rmsnorm_quant(n, h):
     g = _gen(n + h)

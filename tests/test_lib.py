@@ -184,3 +184,27 @@ def test_swiglu_config_choice_by_shape(monkeypatch):
     assert swiglu_config(19456, 2688, 16294) == 30   # 21 K-blocks
     monkeypatch.setenv(SWIGLU_CONFIG_ENV, "10")
     assert swiglu_config(19456, 2560, 16294) == 10
+
+
+def test_swiglu_launches_cover_the_rows(monkeypatch):
+    """gate_up goes out as one launch or as the whole 256-row tiles and the
+    rest: every row once, first rows first, the second launch only where a
+    few rows past a multiple of 256 would cost another round of the CUs; a
+    forced config is one launch."""
+    from quail_amd import engine
+    for env in (engine.SWIGLU_CONFIG_ENV, engine.GEMM_CONFIG_ENV):
+        monkeypatch.delenv(env, raising=False)
+    for n, k in ((19456, 2560), (24576, 4096), (51200, 5120), (256, 128)):
+        for m in (1, 16, 255, 256, 257, 277, 512, 800, 1003, 1300, 4097, 16384):
+            launches = engine.swiglu_launches(n, k, m)
+            assert sum(rows for rows, _ in launches) == m
+            assert len(launches) == 1 or (launches[0][0] % 256 == 0 and launches[0][1] == 30
+                                          and 0 < launches[1][0] < 256)
+            if len(launches) == 1:
+                assert launches[0][1] == engine.swiglu_config(n, k, m)
+    assert engine.swiglu_launches(51200, 5120, 277) == ((256, 30), (21, 48))
+    assert engine.swiglu_launches(19456, 2560, 1003) == ((768, 30), (235, 49))
+    assert len(engine.swiglu_launches(19456, 2560, 277)) == 1
+    assert len(engine.swiglu_launches(19456, 2560, 16384)) == 1
+    monkeypatch.setenv(engine.SWIGLU_CONFIG_ENV, "50")
+    assert engine.swiglu_launches(51200, 5120, 277) == ((277, 50),)
