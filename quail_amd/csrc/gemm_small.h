@@ -11,18 +11,20 @@
 // reads 48 KiB of fragments for 16 KiB of operands) and the direct loads,
 // measured 0.17 (16 x 32) to 0.98 us (256 x 128) a block with one workgroup
 // per CU. With every operand already in L2 the mid tiles run only 5-15%
-// faster, so it is this loop and not the memory that they wait for; the 76
-// gate_up tiles of 256 weight rows are the exception: 12 against 23 us (one
-// CU draws at most 47 GB/s of memory it misses L2 for, 92 of L2 hits).
-//   46 rows, K = 9728, N = 2560:  97 -> 15 us (16 x 32 tiles)
-//   333 rows, same:               98 -> 26 us (64 x 64)
-//   1003 rows, same:              98 -> 47 us (192 x 64)
-//   46 rows, gate_up + SiLU-quant (K = 2560, 2 x 9728): 41 -> 25 us (64 x 256)
+// faster, and a copy of the loads alone draws 120 GB/s per CU from L2 where
+// the tiles draw 41-61, so it is this loop and not the memory that they wait
+// for; the 76 gate_up tiles of 256 weight rows are the exception (12 us with
+// the weights in L2, 23 without).
+//   46 rows, K = 9728, N = 2560:  97 -> 14.5 us (16 x 32 tiles)
+//   333 rows, same:               98 -> 25 us (64 x 64)
+//   1003 rows, same:              98 -> 44 us (192 x 64)
+//   46 rows, gate_up + SiLU-quant (K = 2560, 2 x 9728): 41 -> 24 us (64 x 256)
 // Measured and not kept: weights loaded straight into registers with only
 // the tokens in LDS (1.2-1.5x the time), the K blocks of one tile spread
 // over eight waves whose partials meet in LDS (faster below 8 rows at long
 // K only: 11.8 against 14.1 us at one row), no fragments read ahead, 16
-// waves on the 64- and 128-wide tiles (0.97-1.05x).
+// waves on the 64- and 128-wide tiles (0.97-1.05x), 4 waves (1.2-1.7x), one
+// scale load per stage instead of per block (0.97-1.05x).
 #pragma once
 
 #include "qx_common.h"

@@ -117,7 +117,8 @@ def _wide_tiles_fill_better(n: int, m: int) -> bool:
 # workgroup, of 32 x 32 tiles two). The times are measured on one MI355X over
 # the Qwen3-4B, -8B and -32B projections at 1 to 8192 rows (launches of 60 to
 # 256 tiles, weights not in L2); choosing by them lost 0.1% on average, and
-# 7% at most, against the fastest tile of each of those 348 launches.
+# 7% at most, against the fastest tile of each of those 348 launches. 42, 43,
+# 45 and 46 were measured again with the refill behind the MFMAs.
 PROMOTION_TILES = {
     40: (16, 32, 256, 0.167, 2.9), 41: (32, 32, 512, 0.220, 3.4),
     42: (64, 64, 256, 0.296, 3.8), 43: (128, 64, 256, 0.419, 4.3),
