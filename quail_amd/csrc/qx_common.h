@@ -179,21 +179,21 @@ typedef __attribute__((address_space(3))) uint8_t lds_u8;
 // any later LDS read, including reads of other buffers. Callers order these
 // loads with explicit s_waitcnt vmcnt and barriers. Loads the compiler does
 // not count can only make its own vmcnt waits stricter (vector memory loads
-// complete in order). M0 is overwritten and said to be: nothing that the
-// compiler emits for these kernels keeps a value in it (LDS instructions of
-// this architecture do not read it), and saving and restoring it around each
-// load cost the small GEMM tiles 1-6% (1003 rows of 2560 x 9728: 46.7 -> 44.0
-// us) and the attention of a 2500-row pack 3% (40.8 -> 39.4 us). A kernel
-// uses these loads or the builtin, which sets M0 itself, never both.
+// complete in order). The LDS address is an operand in M0, so the compiler
+// writes that register itself and knows of every use of it; the s_nop is the
+// wait state between that write, which may come right before, and the load.
+// (Written in the assembly and named as a clobber it would be a reserved
+// register, which the compiler does not promise to keep track of; saved and
+// restored around each load it cost the small GEMM tiles 1-6% and the
+// attention of a 2500-row pack 3%.)
 __device__ __forceinline__ void lds_dma16(const void* src, const uint8_t* lds) {
   const uint32_t addr = (uint32_t)(uintptr_t)(lds_u8*)lds;
   asm volatile(
-      "s_mov_b32 m0, %0\n\t"
       "s_nop 1\n\t"
       "global_load_lds_dwordx4 %1, off"
       :
-      : "s"(addr), "v"(src)
-      : "memory", "m0");
+      : "{m0}"(addr), "v"(src)
+      : "memory");
 }
 
 // The same with device scope (sc1: the vector L1 keeps no copy), for
@@ -201,24 +201,22 @@ __device__ __forceinline__ void lds_dma16(const void* src, const uint8_t* lds) {
 __device__ __forceinline__ void lds_dma16_stream(const void* src, const uint8_t* lds) {
   const uint32_t addr = (uint32_t)(uintptr_t)(lds_u8*)lds;
   asm volatile(
-      "s_mov_b32 m0, %0\n\t"
       "s_nop 1\n\t"
       "global_load_lds_dwordx4 %1, off sc1"
       :
-      : "s"(addr), "v"(src)
-      : "memory", "m0");
+      : "{m0}"(addr), "v"(src)
+      : "memory");
 }
 
 // 4 bytes per lane (lane i writes lds + 4 i), untracked like lds_dma16.
 __device__ __forceinline__ void lds_dma4(const void* src, const uint8_t* lds) {
   const uint32_t addr = (uint32_t)(uintptr_t)(lds_u8*)lds;
   asm volatile(
-      "s_mov_b32 m0, %0\n\t"
       "s_nop 1\n\t"
       "global_load_lds_dword %1, off"
       :
-      : "s"(addr), "v"(src)
-      : "memory", "m0");
+      : "{m0}"(addr), "v"(src)
+      : "memory");
 }
 
 // y / s from the hardware reciprocal r = rcp(s) and one FMA correction of

@@ -19,6 +19,29 @@ def test_library_exports_every_declared_symbol():
     assert lib.qx_version() == _lib.ABI_VERSION == _lib.header_abi_version()
 
 
+def test_direct_lds_loads_compile_without_a_warning(tmp_path):
+    """The direct HBM -> LDS loads hand the compiler their M0 operand: named
+    as a clobber instead, M0 is a reserved register the compiler does not
+    keep track of across the statement, and it says so."""
+    from quail_amd import build
+    src = tmp_path / "loads.hip"
+    src.write_text("""
+#include "qx_common.h"
+__global__ void loads(const uint8_t* a, float* out, int n) {
+  __shared__ __attribute__((aligned(1024))) uint8_t buf[3][1024];
+  for (int i = 0; i < n; ++i) {
+    qx::lds_dma16(a + threadIdx.x * 16, buf[0]);
+    qx::lds_dma16_stream(a + 1024 + threadIdx.x * 16, buf[1]);
+    qx::lds_dma4(a + 2048 + threadIdx.x * 4, buf[2]);
+    qx::wait_vmcnt<0>();
+    qx::lds_barrier();
+    out[i * 64 + threadIdx.x] = reinterpret_cast<const float*>(buf)[threadIdx.x * 3];
+  }
+}
+""")
+    assert build._compile(src, tmp_path / "loads.o") == ""
+
+
 def test_argument_errors_return_minus_one_with_a_message():
     with pytest.raises(_lib.QxError, match="null pointer"):
         _lib.call("qx_gemm_fp8_blockscaled", None, None, None, None, None, 1, 256, 128, 128,
