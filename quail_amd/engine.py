@@ -118,17 +118,26 @@ def _wide_tiles_fill_better(n: int, m: int) -> bool:
 # the Qwen3-4B, -8B and -32B projections at 1 to 8192 rows (launches of 60 to
 # 256 tiles, weights not in L2); choosing by them lost 0.1% on average, and
 # 7% at most, against the fastest tile of each of those 348 launches. 42, 43,
-# 45 and 46 were measured again with the refill behind the MFMAs.
+# 45 and 46 were measured again with the refill behind the MFMAs. Over 1152
+# launches of 256 to 10,240 weights, K 128 to 25,600 and 1 to 16,384 rows the
+# choice lost 0.7% on average, and against config 30 or 31 itself more than 2%
+# at two (640 weights x 9728, 16,384 rows: 7%).
 PROMOTION_TILES = {
     40: (16, 32, 256, 0.167, 2.9), 41: (32, 32, 512, 0.220, 3.4),
     42: (64, 64, 256, 0.296, 3.8), 43: (128, 64, 256, 0.419, 4.3),
     44: (192, 64, 256, 0.539, 4.6), 45: (128, 128, 256, 0.560, 6.3),
-    46: (192, 128, 256, 0.750, 7.0), 47: (256, 128, 256, 0.979, 7.9),
+    46: (192, 128, 256, 0.790, 7.0), 47: (256, 128, 256, 0.979, 7.9),
     30: (256, 256, 256, 1.443, 3.9), 31: (256, 320, 256, 1.686, 10.0),
 }
-# the same with the SiLU-quant epilogue
-SWIGLU_TILES = {48: (64, 256, 256, 1.369, -4.0), 49: (96, 256, 256, 1.380, -0.5),
-                50: (128, 256, 256, 1.426, 0.2), 30: (256, 256, 256, 1.933, 1.7)}
+# The same with the SiLU-quant epilogue, a least-squares fit over 1332
+# launches: 512 to 51,200 gate_up rows, K 128 to 5120, 1 to 16,384 rows. No
+# time is below zero, so no K makes another round of the CUs look free: a fit
+# at K >= 2560 alone had -4.0 us besides for 48 and took 64-token tiles for
+# full packs of narrow models (16,384 rows of 19,456 x 256: 322 us, config 30
+# 174). Choosing by these lost 0.02% on average and 4% at most against the
+# fastest tile of each launch.
+SWIGLU_TILES = {48: (64, 256, 256, 0.701, 3.7), 49: (96, 256, 256, 0.905, 4.6),
+                50: (128, 256, 256, 1.025, 5.5), 30: (256, 256, 256, 1.423, 8.1)}
 SWIGLU_SMALL_CONFIGS = (48, 49, 50)
 
 
@@ -203,9 +212,10 @@ def _swiglu_launches(n: int, k: int, m: int) -> tuple:
     rows past a multiple of 256 otherwise cost a whole row of 256 x 256 tiles
     and often another round of the CUs. Measured (us, best one launch / two):
     Qwen3-4B 800 rows 75 / 59, 1003 77 / 66; -8B 1300 rows 162 / 138; -32B 277
-    rows 142 / 129, 800 278 / 258; the table's choice was the faster one, or
-    within 4% of it, at each of 33 sizes from 256 to 1300 rows. The rest costs
-    less than the table says (the first launch leaves its weights in cache)."""
+    rows 142 / 129, 800 278 / 258; the table's choice was the fastest, or
+    within 1% of it, at 151 of 154 sizes (512 to 51,200 gate_up rows, K 128 to
+    5120, 257 to 8300 rows; 6% off at the worst, -32B's 530 rows), and never
+    slower than config 30 in one launch."""
     config = _fastest_tile(n, k, m, True, SWIGLU_DEFAULT_CONFIG)
     first = m // 256 * 256
     if 0 < first < m:

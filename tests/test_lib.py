@@ -198,6 +198,26 @@ def test_promotion_tiles_divide_the_width_and_stay_in_the_family(monkeypatch):
     assert e.gemm_tiles(2560, 9728, 46) == 30
 
 
+def test_tile_costs_rise_with_rows_and_narrow_models_keep_the_large_tile(monkeypatch):
+    """A launch's predicted time is positive and never falls when rows are
+    added, for every tile at every K; full packs run on 256-row tiles also
+    where K is small (a round of the CUs is not free there)."""
+    from quail_amd import engine as e
+    for env in (e.SWIGLU_CONFIG_ENV, e.GEMM_CONFIG_ENV):
+        monkeypatch.delenv(env, raising=False)
+    for table in (e.PROMOTION_TILES, e.SWIGLU_TILES):
+        for tile in table.values():
+            for k in (128, 256, 384, 640, 2560, 25600):
+                costs = [e._tile_cost(tile, 19456 if table is e.SWIGLU_TILES else 2560, k, m)
+                         for m in (1, 64, 65, 257, 1003, 4096, 16384, 1 << 24)]
+                assert costs[0] > 0 and costs == sorted(costs)
+    for n in (2048, 19456, 51200):
+        for k in (128, 256, 640, 2560):
+            assert e.swiglu_config(n, k, 16384) == 30
+            # no launch of millions of one-tile workgroups
+            assert e.swiglu_launches(n, k, 1 << 24) == ((1 << 24, 30),)
+
+
 def test_swiglu_config_choice_by_shape(monkeypatch):
     from quail_amd.engine import GEMM_CONFIG_ENV, SWIGLU_CONFIG_ENV, swiglu_config
     monkeypatch.delenv(GEMM_CONFIG_ENV, raising=False)
