@@ -319,8 +319,8 @@ int qx_paged_attention_qnorm(const void* q, int64_t q_ld, const void* k_pool, co
  * Host function: the query rows per workgroup (work-list tile height) that a
  * paged or LSE call over these sequences runs best with: 32 where
  * qx_paged_attention accepts it and the default-height work items read at
- * most 8 64-key tiles on average (short documents: two 4-wave workgroups per
- * CU hide each other's fixed cost), or many of them are half empty, or their
+ * most 40 64-key tiles on average (two 4-wave workgroups per CU hide each
+ * other's fixed cost and waits), or many of them are half empty, or their
  * workgroups do not outnumber the CUs; else the default. cu_q and used are host copies.
  * Returns the rows or -1. No reference counterpart (FlashAttention's varlen
  * grid has one tile height).

@@ -966,19 +966,23 @@ inline bool attn_rows_ok(int64_t D, int64_t G, int64_t rows) {
   return rows == attn_default_rows(G) || (D == 128 && attn_heads_per_group(G) == 4 && rows == 32);
 }
 
-// The 32-row tile is chosen (both sides measured on one MI355X, 32 heads, 8 KV
-// heads, times of 32 over 64 rows)
+// The 32-row tile is chosen (both sides measured on MI355X, times of 32 over
+// 64 rows; 16,384-row packs, 32 heads and 8 KV heads unless said)
 //   - when the 64-row work items read at most this many 64-key tiles on
-//     average, where two workgroups a CU hide each other's fixed cost: 0.88 on
-//     128-token documents, 0.97 at 512 and 768 tokens; 1.00 at 4096, 1.02 at
-//     8000;
-constexpr double kShortItemTiles = 8.0;
+//     average, where two workgroups a CU hide each other's fixed cost and
+//     waits. Documents of one length, tokens (tiles): 128 (2.5) 0.84, 512
+//     (5.5) 0.98, 768 (7.4) 0.95, 1024 (9.5) 0.96, 1536 (13) 0.98, 2048 (17)
+//     0.98-0.99, 3072 (25) 0.98-0.99, 3600 (28) 0.97, 4096 (33) 1.00-1.01,
+//     5400 (44) 0.985, 8000 (63) 1.005-1.016. Ragged packs, also of 32,768
+//     rows and of 64 heads: 27 to 37 tiles 0.98-1.005, 41 to 50 0.98-1.005,
+//     53 to 65 0.99-1.012. One document of 2112 to 2500 tokens 0.85;
+constexpr double kShortItemTiles = 40.0;
 //   - when the 32-row items together read less than this many times the tiles
 //     of the 64-row ones (2 where every 64-row item is full): the second half
 //     of a 64-row workgroup whose sequence has few rows left works on nothing.
 //     20 documents of ~900 tokens, three 21-row questions on each: 56 us
-//     against 88; 64 of ~300, four 8-row questions: 80 against 155; 48-row
-//     questions (ratio 2): equal;
+//     against 88; 64 of ~300, four 8-row questions: 80 against 155; 48- and
+//     64-row questions (ratio 2) on 800 to 3000 tokens: 0.95-0.98;
 constexpr double kHalfEmptyTiles = 1.7;
 //   - when the 64-row workgroups do not outnumber the CUs: the 32-row ones
 //     then spread one sequence over twice as many. One document of 700

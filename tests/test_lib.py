@@ -82,7 +82,7 @@ def test_attention_work_list_is_heaviest_first_and_covers_every_tile():
 
 def test_attention_tile_rows_choice_and_32_row_work_list():
     """qx_paged_attention_tile_rows picks 32 query rows per workgroup for
-    packs whose 64-row items read few key tiles (at most 8 on average) and
+    packs whose 64-row items read few key tiles (at most 40 on average) and
     the default 64 otherwise; only D = 128 with 4 heads per workgroup offers
     32 (G = 2 keeps its default of 128). A 32-row work list covers every
     32-row tile that holds rows, heaviest first."""
@@ -96,8 +96,10 @@ def test_attention_tile_rows_choice_and_32_row_work_list():
 
     # 512-token documents after a 64-token prefix: 5.5 key tiles per item
     assert rows([512] * 4, [576] * 4) == 32
-    # 1024-token documents: 9.5 key tiles per item
-    assert rows([1024] * 4, [1088] * 4) == 64
+    # 1024- to 4096-token documents: 9.5 to 33.5 key tiles per item, 32-row
+    # workgroups measured up to 5% faster (1.00 at 4096); 8000: 63.5, 1-1.6% slower
+    for n, want in ((1024, 32), (1536, 32), (2048, 32), (4096, 32), (8000, 64)):
+        assert rows([n] * 4, [n + 64] * 4) == want, n
     assert rows([512] * 4, [576] * 4, d=64) == 64
     assert rows([512] * 4, [576] * 4, hq=16, hk=8) == 128
     cu_q = np.array([0, 100, 101, 301], dtype=np.int32)
@@ -131,9 +133,9 @@ def test_attention_tile_rows_for_half_empty_and_few_workgroups():
 
     assert rows([21] * 60, [921] * 60) == 32
     assert rows([21] * 60, [900] * 60, causal=0) == 32
-    assert rows([48] * 240, [2048] * 240) == 64
-    assert rows([2000], [2000]) == 32       # 32 items x 8 head groups = 256 workgroups
-    assert rows([2112], [2112]) == 64
+    assert rows([48] * 240, [4096] * 240) == 64
+    assert rows([2048], [8192]) == 32       # 32 items x 8 head groups = 256 workgroups
+    assert rows([2112], [8192]) == 64
     assert rows([], []) == 64
 
 
