@@ -14,6 +14,8 @@
 //
 // FP8 scales are written "column-major": scale of (token t, group g) at
 // scales[g * s_ld + t], the (K/128, n) storage the reference views as (n, K/128).
+#include <algorithm>
+
 #include "qx_common.h"
 #include "qx_status.h"
 
@@ -234,10 +236,30 @@ __global__ __launch_bounds__(64 * WPR) void norm_quant_row_kernel(
 // 35.5; hidden 5120: 16384 54.7 -> 59.4; hidden 8192: 16384 134 -> 112; MODE
 // 2, hidden 2560: 333 5.6 -> 4.1, 4096 12.6 -> 13.6; hidden 5120: 16384 106.5
 // -> 86.5; hidden 128: 2.8 -> 2.9 at any few rows.
+constexpr bool always_row_workgroups(int niter, int mode) { return niter > (mode == 1 ? 10 : 8); }
+constexpr bool never_row_workgroups(int niter) { return niter < 2; }
 bool row_workgroups(int niter, int mode, int n) {
-  if (niter < 2) return false;
-  if (n <= 1536 || niter > (mode == 1 ? 10 : 8)) return true;
-  return mode == 0 && niter >= 5 && n >= 4096;
+  return n <= 1536 || (mode == 0 && niter >= 5 && n >= 4096);
+}
+
+// One workgroup per row, in launches of fewer than 2^32 threads (more are
+// refused; a wave per row reaches that at 67 M rows, 8 waves at 8.4 M).
+template <int NITER, int MODE>
+void launch_norm_quant_rows(const void* x, int64_t x_ld, void* res, int64_t res_ld,
+                            const int64_t* ids, const void* w, void* q, int64_t q_ld,
+                            float* scales, int64_t s_ld, int n, int H, float eps,
+                            hipStream_t stream) {
+  constexpr int kWaves = NITER <= 8 ? NITER : (NITER + 1) / 2;
+  constexpr int kMaxRows = (int)((1LL << 31) / (64 * kWaves));
+  for (int64_t row = 0; row < n; row += kMaxRows) {
+    const int rows = (int)std::min<int64_t>(n - row, kMaxRows);
+    hipLaunchKernelGGL((norm_quant_row_kernel<NITER, kWaves, MODE>), dim3(rows),
+                       dim3(64 * kWaves), 0, stream,
+                       (const uint16_t*)x + (MODE == 2 ? 0 : row * x_ld), x_ld,
+                       MODE == 1 ? nullptr : (uint16_t*)res + row * res_ld, res_ld,
+                       MODE == 2 ? ids + row : nullptr, (const uint16_t*)w,
+                       (uint8_t*)q + row * q_ld, q_ld, scales + row, s_ld, H, eps);
+  }
 }
 
 template <int MODE>
@@ -246,20 +268,20 @@ int launch_norm_quant(const void* x, int64_t x_ld, void* res, int64_t res_ld, co
                       int H, float eps, hipStream_t stream) {
   const int niter = (H / 8 + 63) / 64;
   dim3 grid((n + 3) / 4), block(kRowThreads);
+  QX_CHECK(n >= 0, "norm_quant: %d rows", n);
 #define QX_NQ_CASE(NI)                                                                     \
-  case NI: {                                                                               \
-    constexpr int kWaves = NI <= 8 ? NI : (NI + 1) / 2;                                    \
-    if (row_workgroups(NI, MODE, n))                                                       \
-      hipLaunchKernelGGL((norm_quant_row_kernel<NI, kWaves, MODE>), dim3(n),               \
-                         dim3(64 * kWaves), 0, stream, (const uint16_t*)x, x_ld,           \
-                         (uint16_t*)res, res_ld, ids, (const uint16_t*)w, (uint8_t*)q,     \
-                         q_ld, scales, s_ld, H, eps);                                      \
-    else                                                                                   \
+  case NI:                                                                                 \
+    if constexpr (!never_row_workgroups(NI))                                               \
+      if (always_row_workgroups(NI, MODE) || row_workgroups(NI, MODE, n)) {                \
+        launch_norm_quant_rows<NI, MODE>(x, x_ld, res, res_ld, ids, w, q, q_ld, scales,    \
+                                         s_ld, n, H, eps, stream);                         \
+        break;                                                                             \
+      }                                                                                    \
+    if constexpr (!always_row_workgroups(NI, MODE))                                        \
       hipLaunchKernelGGL((norm_quant_kernel<NI, MODE>), grid, block, 0, stream,            \
                          (const uint16_t*)x, x_ld, (uint16_t*)res, res_ld, ids,            \
                          (const uint16_t*)w, (uint8_t*)q, q_ld, scales, s_ld, n, H, eps);  \
-    break;                                                                                 \
-  }
+    break;
   switch (niter) {
     QX_NQ_CASE(1)
     QX_NQ_CASE(2)

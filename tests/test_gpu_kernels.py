@@ -485,6 +485,39 @@ def test_norm_quant_rows_do_not_depend_on_how_many_share_the_launch(h):
             assert torch.equal(a, b[rows])
 
 
+def test_norm_quant_of_more_rows_than_one_launch_holds():
+    """A workgroup of six waves per row reaches a launch's 2^32 threads at
+    11.2 M rows: such a call goes out in several launches. Every row reads one
+    and the same input row and writes one and the same code row (strides of
+    0), each its own scales; the last row's id selects another row where the
+    embedding form has ids."""
+    from quail_amd import _lib
+    h, n = 5248, (1 << 32) // (6 * 64) + 7
+    g = _gen(77)
+    x = torch.randn(2, h, generator=g).to(torch.bfloat16).to(DEV)
+    w = (1 + 0.1 * torch.randn(h, generator=g)).to(torch.bfloat16).to(DEV)
+    eng = _engine(4, 2, 64)
+    norm = type("N", (), {"weight": w, "variance_epsilon": 1e-6})()
+    want_q, want_s = eng.norm_quant(x, norm)
+    q = torch.zeros(h, dtype=torch.uint8, device=DEV)
+    s = torch.zeros(h // 128, n, device=DEV)
+    _lib.call("qx_rmsnorm_quant", _ptr(x), 0, _ptr(w), _ptr(q), 0, _ptr(s), n, n, h, 1e-6,
+              _stream())
+    assert torch.equal(q, want_q[0].view(torch.uint8))
+    assert torch.equal(s, want_s[0][:, None].expand(-1, n))
+    s.zero_()
+    res = torch.zeros(h, dtype=torch.bfloat16, device=DEV)
+    ids = torch.zeros(n, dtype=torch.int64, device=DEV)
+    ids[-1] = 1
+    _lib.call("qx_embed_rmsnorm_quant", _ptr(x), h, _ptr(ids), _ptr(res), 0, _ptr(w), _ptr(q), 0,
+              _ptr(s), n, n, h, 1e-6, _stream())
+    assert torch.equal(s[:, :-1], want_s[0][:, None].expand(-1, n - 1))
+    assert torch.equal(s[:, -1], want_s[1])
+    with pytest.raises(_lib.QxError):
+        _lib.call("qx_rmsnorm_quant", _ptr(x), 0, _ptr(w), _ptr(q), 0, _ptr(s), n, -3, h, 1e-6,
+                  _stream())
+
+
 @pytest.mark.parametrize("n,h", [(3, 256), (64, 2560)])
 def test_rmsnorm_quant_and_embed_fused(n, h):
     g = _gen(7 * n + h)
