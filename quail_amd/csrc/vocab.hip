@@ -14,10 +14,12 @@
 //     to a per-token (max, sum of exp) partial; the waves' partials merge
 //     in LDS into one per (head-row block, token). The lane holding a target
 //     id's logit writes it.
-//   * vocab_finish_kernel: one wave per token merges the blocks' partials
-//     into the logsumexp and subtracts it from the target logits.
+//   * vocab_finish_kernel: a workgroup of 8 waves per token merges the
+//     blocks' partials into the logsumexp (the waves' through LDS) and
+//     subtracts it from the target logits.
 // The head (V x H bf16, 778 MB for Qwen3) is read once per 128 tokens, so a
 // launch over a pack's final rows is bound by streaming it from HBM.
+#include <algorithm>
 #include <mutex>
 
 #include "qx_common.h"
@@ -206,11 +208,11 @@ constexpr int kFinishThreads = 512;
 
 __global__ __launch_bounds__(kFinishThreads) void vocab_finish_kernel(
     const float2* __restrict__ part, int nblk, const float* __restrict__ tlogit, int t,
-    float* __restrict__ out, int64_t out_ld, int n) {
+    float* __restrict__ out, int64_t out_ld, int n, int tok0) {
   constexpr int kAhead = 4;
   constexpr int kFinishWaves = kFinishThreads / 64;
   __shared__ float2 red[kFinishWaves];
-  const int tok = blockIdx.x;
+  const int tok = tok0 + blockIdx.x;
   const int lane = threadIdx.x & 63;
   float target = 0.0f;
   if ((int)threadIdx.x < t) target = tlogit[(int64_t)tok * t + threadIdx.x];
@@ -300,8 +302,12 @@ int vocab_run(const void* normed, int64_t n_ld, const void* head, int64_t h_ld,
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
   }
-  hipLaunchKernelGGL(vocab_finish_kernel, dim3((unsigned)n), dim3(kFinishThreads), 0,
-                     stream, part, nblk, tlogit, (int)t, out, out_ld, (int)n);
+  // launches of fewer than 2^32 threads: past that the grid wraps around
+  constexpr int64_t kMaxTokens = (1LL << 31) / kFinishThreads;
+  for (int64_t tok = 0; tok < n; tok += kMaxTokens)
+    hipLaunchKernelGGL(vocab_finish_kernel, dim3((unsigned)std::min(n - tok, kMaxTokens)),
+                       dim3(kFinishThreads), 0, stream, part, nblk, tlogit, (int)t, out, out_ld,
+                       (int)n, (int)tok);
   QX_LAUNCH_STATUS();
 }
 

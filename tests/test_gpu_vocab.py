@@ -58,6 +58,23 @@ def test_vocab_logprobs_match_float64(n, vocab, hidden):
     assert torch.equal(got[:, 1], got[:, 4])
 
 
+def test_vocab_logprobs_of_more_rows_than_one_merge_launch_holds():
+    """8.4 M rows: a workgroup of 512 threads per row is past a launch's 2^32
+    threads; every 997th row and the last ones are what few rows give."""
+    n, vocab, hidden = (1 << 23) + 9, 130, 64
+    normed, head = _case(n, vocab, hidden, seed=5)
+    t = torch.tensor([0, 129], dtype=torch.long, device=DEV)
+    got = torch.empty(n, 2, device=DEV)
+    size = _lib.count("qx_vocab_logprobs_workspace", n, vocab, 2)
+    ws = torch.empty(size, dtype=torch.uint8, device=DEV)
+    _lib.call("qx_vocab_logprobs", normed.data_ptr(), hidden, head.data_ptr(), hidden,
+              t.data_ptr(), 2, got.data_ptr(), 2, n, vocab, hidden, ws.data_ptr(), size,
+              torch.cuda.current_stream().cuda_stream)
+    readout = AsyncLabelLogprobs(head, [0, 129], normalize=True)
+    for rows in (slice(0, n, 997), slice(n - 300, n)):
+        assert torch.equal(got[rows], readout.logprobs(normed[rows].contiguous()))
+
+
 def test_normalized_minus_logits_is_the_row_logsumexp():
     """normalize=True minus normalize=False (the targets' bf16 logits) is one
     number per row, -logsumexp, for every target."""
