@@ -53,16 +53,24 @@ GEMM_ODD_WIDTH_CONFIG = 11
 CUS = 256
 
 
-_environ = getattr(os.environ, "_data", None)   # the dict os.environ wraps
+_Environ = type(os.environ)
 
 
 def _forced(name):
-    """os.environ.get(name). Each GEMM asks; os.environ encodes the name and
-    raises and catches KeyError every time (1.6 us against 0.2)."""
-    if type(_environ) is not dict or os.name != "posix":
-        return os.environ.get(name)
-    value = _environ.get(name.encode())
-    return None if value is None else os.fsdecode(value)
+    """os.environ.get(name) of what os.environ is at the call. Each GEMM asks,
+    and Python's own environment mapping raises and catches KeyError for every
+    name that is not set (0.9 us against 0.4): its dict is asked instead,
+    where it has one. Any other mapping in its place is asked as it is."""
+    env = os.environ
+    data = getattr(env, "_data", None) if type(env) is _Environ else None
+    if type(data) is not dict:
+        return env.get(name)
+    value = data.get(env.encodekey(name))
+    return None if value is None else env.decodevalue(value)
+
+
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", None)
 
 
 def _ptr(t):
@@ -71,8 +79,11 @@ def _ptr(t):
 
 def _stream():
     """The handle of the current stream of the current device (without the
-    Stream object torch.cuda.current_stream() makes around it)."""
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    Stream object torch.cuda.current_stream() makes around it, where this
+    torch has the functions it is made from)."""
+    if _raw_stream is None or _current_device is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_current_device())
 
 
 def gemm_config(n: int, k: int, m: int) -> int:
@@ -80,7 +91,7 @@ def gemm_config(n: int, k: int, m: int) -> int:
     family for widths that are a multiple of 256 or 320 (256 x 320 tiles
     where they take fewer full-wave units, or where 256 x 256 ones cannot
     tile N), config 11 for the rest."""
-    forced = os.environ.get(GEMM_CONFIG_ENV)
+    forced = _forced(GEMM_CONFIG_ENV)
     return _family_config(n, m) if forced is None else int(forced)
 
 

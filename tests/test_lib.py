@@ -231,6 +231,40 @@ def test_swiglu_config_choice_by_shape(monkeypatch):
     assert swiglu_config(19456, 2560, 16294) == 10
 
 
+def test_forced_configs_are_read_from_the_environment_of_the_call(monkeypatch):
+    """A forced config is seen wherever the program put it: os.environ set
+    after the import, another mapping in os.environ's place, and that
+    mapping's own changes; without it the choice is the table's."""
+    import os
+
+    from quail_amd import engine as e
+    for env in (e.SWIGLU_CONFIG_ENV, e.GEMM_CONFIG_ENV):
+        monkeypatch.delenv(env, raising=False)
+    assert e.gemm_tiles(2560, 9728, 46) == 40
+    monkeypatch.setenv(e.GEMM_CONFIG_ENV, "30")
+    assert e.gemm_tiles(2560, 9728, 46) == e.gemm_config(2560, 9728, 46) == 30
+    assert e.swiglu_launches(19456, 2560, 1003) == ((1003, 30),)
+    mine = {e.GEMM_CONFIG_ENV: "42"}
+    monkeypatch.setattr(os, "environ", mine)
+    assert e.gemm_tiles(2560, 9728, 46) == e.gemm_config(2560, 9728, 46) == 42
+    mine[e.SWIGLU_CONFIG_ENV] = "50"
+    assert e.swiglu_config(19456, 2560, 46) == 50
+    mine.clear()
+    assert e.gemm_tiles(2560, 9728, 46) == 40
+
+
+def test_stream_handle_where_torch_lacks_the_raw_one(monkeypatch):
+    """The launch stream is torch's current one, also in a torch without the
+    functions that give its handle alone."""
+    import torch
+
+    from quail_amd import engine as e
+    stream = type("Stream", (), {"cuda_stream": 1234})()
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: stream)
+    monkeypatch.setattr(e, "_raw_stream", None)
+    assert e._stream() == 1234
+
+
 def test_swiglu_launches_cover_the_rows(monkeypatch):
     """gate_up goes out as one launch or as the whole 256-row tiles and the
     rest: every row once, first rows first, the second launch only where a
