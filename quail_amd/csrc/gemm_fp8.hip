@@ -198,29 +198,8 @@ __device__ __forceinline__ void tile_epilogue(uint8_t* smem, const v16f (&acc)[T
       const int row = wave * kRowsPerWave + i * 4 + (lane >> 4);
       const int m = m0 + row;
       const uint8_t* lrow = smem + row * kRowBytes;
-      const uint4 g = *reinterpret_cast<const uint4*>(lrow + seg * 16);
-      const uint4 u = *reinterpret_cast<const uint4*>(lrow + 256 + seg * 16);
-      const uint32_t gw[4] = {g.x, g.y, g.z, g.w}, uw[4] = {u.x, u.y, u.z, u.w};
-      float y[8];
-      float amax = 0.0f;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        y[2 * k] = silu_mul(lo_bf16(gw[k]), lo_bf16(uw[k]));
-        y[2 * k + 1] = silu_mul(hi_bf16(gw[k]), hi_bf16(uw[k]));
-      }
-#pragma unroll
-      for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(y[k]));
-      amax = group_max<16>(amax);
-      const float scale = fp8_scale(amax);
-      const float rs = recip(scale);
-      if (m < M) {
-        const v2i o = {(int)pack4_fp8(silu_quot(y[0], rs), silu_quot(y[1], rs),
-                                      silu_quot(y[2], rs), silu_quot(y[3], rs)),
-                       (int)pack4_fp8(silu_quot(y[4], rs), silu_quot(y[5], rs),
-                                      silu_quot(y[6], rs), silu_quot(y[7], rs))};
-        __builtin_nontemporal_store(o, reinterpret_cast<v2i*>(Q + (int64_t)m * q_ld + j0 + seg * 8));
-        if (seg == 0) Qs[(int64_t)(j0 >> 7) * qs_ld + m] = scale;
-      }
+      swiglu_quant_row<true>(lrow, seg, m < M, Q + (int64_t)m * q_ld + j0 + seg * 8,
+                             Qs + (int64_t)(j0 >> 7) * qs_ld + m);
     }
   } else {
     constexpr int kRowsPerOp = 64 / kChunks;
@@ -907,30 +886,8 @@ __global__ __launch_bounds__(512) void gemm_fp8_k128q_kernel(
           const int prow = wave * kRowsPerWave + i * 4 + (lane >> 4);
           const int m = m0 + (prow >> 5) * TM * 32 + b * 32 + (prow & 31);
           const uint8_t* lrow = buf + prow * kRowBytes;
-          const uint4 g = *reinterpret_cast<const uint4*>(lrow + seg * 16);
-          const uint4 u = *reinterpret_cast<const uint4*>(lrow + 256 + seg * 16);
-          const uint32_t gw[4] = {g.x, g.y, g.z, g.w}, uw[4] = {u.x, u.y, u.z, u.w};
-          float y[8];
-          float amax = 0.0f;
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            y[2 * k] = silu_mul(lo_bf16(gw[k]), lo_bf16(uw[k]));
-            y[2 * k + 1] = silu_mul(hi_bf16(gw[k]), hi_bf16(uw[k]));
-          }
-#pragma unroll
-          for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(y[k]));
-          amax = group_max<16>(amax);
-          const float scale = fp8_scale(amax);
-          const float rs = recip(scale);
-          if (m < M) {
-            const v2i o = {(int)pack4_fp8(silu_quot(y[0], rs), silu_quot(y[1], rs),
-                                          silu_quot(y[2], rs), silu_quot(y[3], rs)),
-                           (int)pack4_fp8(silu_quot(y[4], rs), silu_quot(y[5], rs),
-                                          silu_quot(y[6], rs), silu_quot(y[7], rs))};
-            __builtin_nontemporal_store(o, reinterpret_cast<v2i*>(Q + (int64_t)m * q_ld + j0 +
-                                                                 seg * 8));
-            if (seg == 0) Qs[(int64_t)(j0 >> 7) * qs_ld + m] = scale;
-          }
+          swiglu_quant_row<true>(lrow, seg, m < M, Q + (int64_t)m * q_ld + j0 + seg * 8,
+                                 Qs + (int64_t)(j0 >> 7) * qs_ld + m);
         }
       } else {
         constexpr int kChunks = BN / 8;
@@ -1350,30 +1307,8 @@ __global__ __launch_bounds__(512) void gemm_fp8_promo_kernel(
           const int prow = wave * kRowsPerWave + i * 4 + (lane >> 4);
           const int m = m0 + (prow >> 5) * TM * 16 + pass * 32 + (prow & 31);  // kTPP = 2
           const uint8_t* lrow = buf + prow * kRowBytes;
-          const uint4 g = *reinterpret_cast<const uint4*>(lrow + seg * 16);
-          const uint4 u = *reinterpret_cast<const uint4*>(lrow + 256 + seg * 16);
-          const uint32_t gw[4] = {g.x, g.y, g.z, g.w}, uw[4] = {u.x, u.y, u.z, u.w};
-          float y[8];
-          float amax = 0.0f;
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            y[2 * k] = silu_mul(lo_bf16(gw[k]), lo_bf16(uw[k]));
-            y[2 * k + 1] = silu_mul(hi_bf16(gw[k]), hi_bf16(uw[k]));
-          }
-#pragma unroll
-          for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(y[k]));
-          amax = group_max<16>(amax);
-          const float scale = fp8_scale(amax);
-          const float rs = recip(scale);
-          if (m < M) {
-            const v2i o = {(int)pack4_fp8(silu_quot(y[0], rs), silu_quot(y[1], rs),
-                                          silu_quot(y[2], rs), silu_quot(y[3], rs)),
-                           (int)pack4_fp8(silu_quot(y[4], rs), silu_quot(y[5], rs),
-                                          silu_quot(y[6], rs), silu_quot(y[7], rs))};
-            __builtin_nontemporal_store(o, reinterpret_cast<v2i*>(Q + (int64_t)m * q_ld + j0 +
-                                                                 seg * 8));
-            if (seg == 0) Qs[(int64_t)(j0 >> 7) * qs_ld + m] = scale;
-          }
+          swiglu_quant_row<true>(lrow, seg, m < M, Q + (int64_t)m * q_ld + j0 + seg * 8,
+                                 Qs + (int64_t)(j0 >> 7) * qs_ld + m);
         }
       } else {
         // 16-byte chunks of the wave's staged rows, 64 per store instruction

@@ -59,35 +59,14 @@ __device__ __forceinline__ void swiglu_quant_rows(const uint8_t* smem, int wave,
                                                   int j0, int M, uint8_t* __restrict__ Q,
                                                   int64_t q_ld, float* __restrict__ Qs,
                                                   int64_t qs_ld) {
-          const int seg = lane & 15;
-      for (int g4 = wave; g4 < BM / 4; g4 += NW) {
-        const int prow = g4 * 4 + (lane >> 4);
-        const int m = m0 + prow;
-        const uint8_t* lrow = smem + prow * kSwigluRow;
-        const uint4 g = *reinterpret_cast<const uint4*>(lrow + seg * 16);
-        const uint4 u = *reinterpret_cast<const uint4*>(lrow + 256 + seg * 16);
-        const uint32_t gw[4] = {g.x, g.y, g.z, g.w}, uw[4] = {u.x, u.y, u.z, u.w};
-        float y[8];
-        float amax = 0.0f;
-  #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          y[2 * k] = silu_mul(lo_bf16(gw[k]), lo_bf16(uw[k]));
-          y[2 * k + 1] = silu_mul(hi_bf16(gw[k]), hi_bf16(uw[k]));
-        }
-  #pragma unroll
-        for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(y[k]));
-        amax = group_max<16>(amax);
-        const float scale = fp8_scale(amax);
-        const float rs = recip(scale);
-        if (m < M) {
-          const v2i o = {(int)pack4_fp8(silu_quot(y[0], rs), silu_quot(y[1], rs),
-                                        silu_quot(y[2], rs), silu_quot(y[3], rs)),
-                         (int)pack4_fp8(silu_quot(y[4], rs), silu_quot(y[5], rs),
-                                        silu_quot(y[6], rs), silu_quot(y[7], rs))};
-          *reinterpret_cast<v2i*>(Q + (int64_t)m * q_ld + j0 + seg * 8) = o;
-          if (seg == 0) Qs[(int64_t)(j0 >> 7) * qs_ld + m] = scale;
-        }
-      }
+  const int seg = lane & 15;
+  for (int g4 = wave; g4 < BM / 4; g4 += NW) {
+    const int prow = g4 * 4 + (lane >> 4);
+    const int m = m0 + prow;
+    swiglu_quant_row<false>(smem + prow * kSwigluRow, seg, m < M,
+                            Q + (int64_t)m * q_ld + j0 + seg * 8,
+                            Qs + (int64_t)(j0 >> 7) * qs_ld + m);
+  }
 }
 
 // BM tokens x BN weights by WM x WN waves; the operands of KPB 128-K blocks

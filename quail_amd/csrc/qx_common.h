@@ -311,6 +311,43 @@ __device__ __forceinline__ float fp8_scale(float amax) {
   return (q0 == __builtin_inff() ? q0 : q) * 0.015625f;
 }
 
+// The gate_up GEMMs' epilogue on one row of a tile staged in LDS, 128 gate
+// then 128 up bf16: 16 lanes (seg 0 to 15) form the row's 128 SiLU-gated
+// products, one quant group; each writes its 8 codes to q (STREAM: past the
+// caches) and the first its scale, where the row exists. One definition, so
+// that every tile shape gives the same bits.
+template <bool STREAM>
+__device__ __forceinline__ void swiglu_quant_row(const uint8_t* lrow, int seg, bool live,
+                                                 uint8_t* q, float* scale_out) {
+  const uint4 g = *reinterpret_cast<const uint4*>(lrow + seg * 16);
+  const uint4 u = *reinterpret_cast<const uint4*>(lrow + 256 + seg * 16);
+  const uint32_t gw[4] = {g.x, g.y, g.z, g.w}, uw[4] = {u.x, u.y, u.z, u.w};
+  float y[8];
+  float amax = 0.0f;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    y[2 * k] = silu_mul(lo_bf16(gw[k]), lo_bf16(uw[k]));
+    y[2 * k + 1] = silu_mul(hi_bf16(gw[k]), hi_bf16(uw[k]));
+  }
+#pragma unroll
+  for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(y[k]));
+  amax = group_max<16>(amax);
+  const float scale = fp8_scale(amax);
+  const float rs = recip(scale);
+  if (live) {
+    const v2i o = {(int)pack4_fp8(silu_quot(y[0], rs), silu_quot(y[1], rs), silu_quot(y[2], rs),
+                                  silu_quot(y[3], rs)),
+                   (int)pack4_fp8(silu_quot(y[4], rs), silu_quot(y[5], rs), silu_quot(y[6], rs),
+                                  silu_quot(y[7], rs))};
+    if constexpr (STREAM) {
+      __builtin_nontemporal_store(o, reinterpret_cast<v2i*>(q));
+    } else {
+      *reinterpret_cast<v2i*>(q) = o;
+    }
+    if (seg == 0) *scale_out = scale;
+  }
+}
+
 }  // namespace qx
 
 // Status codes of every extern "C" entry point.
