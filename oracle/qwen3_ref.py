@@ -194,7 +194,7 @@ def paged_attention(q3, k_pool, v_pool, cu_q, used, table, page, causal=True, sc
             continue
         pages = [int(p) for p in table[s][: -(-seen // page)]]
         rows = torch.tensor([p * page + j for p in pages for j in range(page)],
-                            device=k_pool.device)[:seen]
+                            dtype=torch.long, device=k_pool.device)[:seen]
         k = k_pool[rows].to(ACCUM).repeat_interleave(group, dim=1)   # (seen, H, D)
         v = v_pool[rows].to(ACCUM).repeat_interleave(group, dim=1)
         qs = q3[r0:r1].to(ACCUM)                                     # (q_len, H, D)

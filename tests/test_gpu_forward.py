@@ -314,3 +314,79 @@ def test_read_rows_answers_equal_those_rows_of_read_all(mode):
     assert len(final) == 3 * 5 and got.shape[0] == len(final)
     pick = [all_final.index(r) for r in final]
     assert torch.equal(got, all_rows[pick])
+
+
+@pytest.mark.parametrize("mode", ["unified", "tree"])
+def test_whole_pass_is_the_same_bits_under_other_tiles_and_tile_heights(mode, monkeypatch):
+    """Three layers of the Qwen3-4B sizes over a pack of some 1000 rows
+    (unified: four documents, one answer row each; tree: the same with label
+    paths),
+    once as the engine picks (small GEMM tiles, gate_up in two launches,
+    32-row attention workgroups) and once with every GEMM on 256 x 256 tiles
+    and attention work lists of the default height: the final rows and every
+    page of every layer are the same bits."""
+    import dataclasses
+
+    from quail_amd import chunk as ch, engine
+    from quail_amd import labels as trie
+    from quail_amd.arena import KVArena
+    from quail_amd.qwen3 import Qwen3Pipeline
+
+    for env in (engine.GEMM_CONFIG_ENV, engine.SWIGLU_CONFIG_ENV):
+        monkeypatch.delenv(env, raising=False)
+    cfg = dataclasses.replace(CONFIGS["qwen3-4b"], layers=3, vocab=512)
+    model = build_synthetic(cfg, seed=4, device="cuda", norm_init="random")
+    labels = [(100, 7), (100, 8, 9), (101, 4), (101, 5), (102, 3)]
+    read = trie.read_nodes(labels)
+    paths = trie.trie_paths(labels, read)
+    mask = trie.path_reads(paths, read)
+    lens = [460, 33, 440, 62]
+    real_work_list = ch._work_list
+
+    def one_pass(plain):
+        rng = np.random.default_rng(8)
+        ids = lambda n: rng.integers(0, cfg.vocab, n, dtype=np.int64)  # noqa: E731
+        arena = KVArena(cfg.layers, 128, 16, cfg.kv_heads, cfg.head_dim)
+        for k, v in zip(arena.k, arena.v):
+            k.zero_()
+            v.zero_()
+        groups, prefix = [], 32
+        for d, n in enumerate(lens):
+            start = prefix if d else 0
+            arena.alloc(("doc", d), n + start, capacity_tokens=n + start + 1,
+                        borrow=(("doc", 0), start) if start else None)
+            g = dict(key=("doc", d), prefix=ids(n), f=n + start, start=start, suffixes=[ids(1)])
+            if mode == "tree":
+                g.update(suffixes=[trie.path_tokens(paths, 1)], paths=paths, read_mask=mask,
+                         read_all_rows=True)
+            groups.append(g)
+        heights = []
+
+        def work_list(tables, heads, choose_rows=False):
+            out = real_work_list(tables, heads, choose_rows=choose_rows and not plain)
+            heights.append(out[2])
+            return out
+
+        with monkeypatch.context() as m:
+            m.setattr(ch, "_work_list", work_list)
+            if plain:
+                m.setenv(engine.GEMM_CONFIG_ENV, "30")
+            chunk = ch.pack_chunk(arena, groups, attention_mode=mode,
+                                  attention_heads=(cfg.heads, cfg.kv_heads, cfg.head_dim))
+            # the engine's own choices are other ones than the plain pass's
+            assert (32 in heights) != plain
+            if not plain:
+                launches = engine.swiglu_launches(2 * cfg.intermediate, cfg.hidden, chunk.tokens)
+                assert len(launches) == 2
+                assert engine.gemm_tiles(cfg.hidden, cfg.intermediate, chunk.tokens) >= 40
+            up = ch.upload(chunk, ch.InputStaging())
+            normed = Qwen3Pipeline(model, arena).forward_chunk(up)
+            torch.cuda.synchronize()
+        return normed, arena
+
+    (a, arena_a), (b, arena_b) = one_pass(False), one_pass(True)
+    assert a.shape[0] >= len(lens) and torch.equal(a, b)
+    assert bool(torch.isfinite(a.float()).all())
+    for layer in range(cfg.layers):
+        for x, y in zip(arena_a.layer_kv(layer), arena_b.layer_kv(layer)):
+            assert torch.equal(x, y) and bool((x != 0).any())

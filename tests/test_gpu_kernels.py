@@ -200,15 +200,25 @@ def test_gemm_promotion_tile_boundaries_with_few_blocks(m, n, k, monkeypatch):
         _bf16_close(outs[PROMOTION_WIDE_CONFIG][rows], ref.gemm(q[rows], s[rows], lin))
 
 
-@pytest.mark.parametrize("m,n,k", [(1, 640, 256), (300, 640, 512), (700, 1920, 1152)])
+@pytest.mark.parametrize("m,n,k", [(1, 640, 256), (300, 640, 512), (700, 1920, 1152),
+                                   (16385, 640, 256)])
 def test_gemm_wide_promotion_tiles_at_widths_only_320_divides(m, n, k, monkeypatch):
-    """Widths that are multiples of 320 but not of 256 take config 31 (the
-    engine's choice) and agree with the oracle to the bf16 tolerance."""
-    from quail_amd.engine import gemm_config
+    """Widths that are multiples of 320 but not of 256 take config 31's tiles
+    where there are many rows and smaller ones for few: config 31 agrees with
+    the oracle to the bf16 tolerance and gives the bits of the engine's own
+    choice, which it is at 16,385 rows (checked on the first and last rows)."""
+    from quail_amd.engine import gemm_config, gemm_tiles
     monkeypatch.delenv("QUAIL_GEMM_CONFIG", raising=False)
     assert gemm_config(n, k, m) == PROMOTION_WIDE_CONFIG
+    assert (gemm_tiles(n, k, m) == PROMOTION_WIDE_CONFIG) == (m > 16384)
     q, s, wq, ws = _gemm_case(m, n, k, seed=m + n + k)
-    _bf16_close(_run_gemm(q, s, wq, ws), ref.gemm(q, s, ref.RefLinear(wq, ws)))
+    picked = _run_gemm(q, s, wq, ws).cpu()
+    monkeypatch.setenv("QUAIL_GEMM_CONFIG", str(PROMOTION_WIDE_CONFIG))
+    wide = _run_gemm(q, s, wq, ws).cpu()
+    assert torch.equal(picked, wide)
+    lin = ref.RefLinear(wq, ws)
+    for rows in (slice(0, 700), slice(max(0, m - 700), m)):
+        _bf16_close(wide[rows], ref.gemm(q[rows], s[rows], lin))
 
 
 SMALL_TILES = {40: (16, 32), 41: (32, 32), 42: (64, 64), 43: (128, 64), 44: (192, 64),
@@ -459,9 +469,11 @@ def test_add_rmsnorm_quant(n, h):
 
 @pytest.mark.parametrize("h", [384, 640, 2560, 4096, 5120, 8192])
 def test_norm_quant_rows_do_not_depend_on_how_many_share_the_launch(h):
-    """Rows of launches whose rows have a wave each (1537 rows; 2048 to 4095
-    with a residual) are the same bits as alone, where a row has a workgroup
-    of its own, in all three forms."""
+    """Rows of launches whose rows have a wave each are the same bits as
+    alone, where a row has a workgroup of its own: 1537 rows of at most 4096
+    columns in all three forms, of 5120 in the one without a residual and
+    without ids. (The other forms of 5120 and all of 8192 columns always have
+    a workgroup per row: test_norm_quant_of_wide_rows_matches_the_oracle.)"""
     g = _gen(h)
     eng = _engine(4, 2, 64)
     n = 1537
@@ -483,6 +495,33 @@ def test_norm_quant_rows_do_not_depend_on_how_many_share_the_launch(h):
     for rows in (slice(0, 1), slice(700, 737), slice(n - 1, n), slice(1, n)):
         for a, b in zip(forms(rows), whole):
             assert torch.equal(a, b[rows])
+
+
+@pytest.mark.parametrize("h", [4224, 5120, 5248, 8192])
+@pytest.mark.parametrize("n", [3, 40])
+def test_norm_quant_of_wide_rows_matches_the_oracle(n, h):
+    """All three forms at the widths whose rows always have a workgroup of
+    their own (two passes per wave; 4224 and 5248 with a partial last pass):
+    the oracle's codes, scales and residual rows."""
+    g = _gen(n + h)
+    eng = _engine(4, 2, 64)
+    x = torch.randn(n, h, generator=g).to(torch.bfloat16)
+    res = torch.randn(n, h, generator=g).to(torch.bfloat16)
+    w = (1 + 0.1 * torch.randn(h, generator=g)).to(torch.bfloat16)
+    norm = type("N", (), {"weight": w.to(DEV), "variance_epsilon": 1e-6})()
+    res_d = res.to(DEV)
+    q, s = eng.norm_quant(x.to(DEV), norm, res_d)
+    q_ref, s_ref, res_ref = ref.add_rms_norm_quant(x, res, w, 1e-6)
+    assert torch.equal(res_d.cpu(), res_ref)
+    _fp8_close(q, s, q_ref, s_ref)
+    q, s = eng.norm_quant(x.to(DEV), norm)
+    q_ref, s_ref = ref.norm_quant_first(x, w, 1e-6)
+    _fp8_close(q, s, q_ref, s_ref)
+    ids = torch.randint(0, n, (n,), generator=g)
+    q, s, rows = eng.embed_norm_quant(ids.to(DEV), x.to(DEV), norm)
+    assert torch.equal(rows.cpu(), x[ids])
+    q_ref, s_ref = ref.norm_quant_first(x[ids], w, 1e-6)
+    _fp8_close(q, s, q_ref, s_ref)
 
 
 def test_norm_quant_of_more_rows_than_one_launch_holds():
@@ -889,7 +928,8 @@ def test_paged_attention_32_row_workgroups_are_bit_identical(v_dtype):
 @pytest.mark.parametrize("rows", [0, 32])
 @pytest.mark.parametrize("v_dtype", V_DTYPES)
 def test_paged_attention_around_its_tile_counts(rows, v_dtype):
-    """Sequences of zero to seven 64-key tiles, each with its last tile whole,
+    """Sequences of zero to eight 64-key tiles (63 to 449 keys; a row that
+    sees no key, and a sequence without rows), each with its last tile whole,
     one key short and one key over (the pipeline's steps with loads spread
     over the MFMAs take whole tiles only, three ahead; the last steps take
     the rest), with one query row and with more rows than a workgroup holds:
@@ -904,6 +944,9 @@ def test_paged_attention_around_its_tile_counts(rows, v_dtype):
             for q_len in (1, min(keys, 67)):
                 used.append(keys)
                 q_lens.append(q_len)
+    for at, q_len in ((5, 0), (9, 1)):
+        used.insert(at, 0)
+        q_lens.insert(at, q_len)
     rng = np.random.default_rng(17)
     pages = [-(-u // page) for u in used]
     perm = rng.permutation(sum(pages) + 9)
