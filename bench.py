@@ -207,7 +207,7 @@ def gemm_alone(reps: int = 20, seed: int = 0):
     on the launch stream after 3 untimed ones. Returns the sub-record."""
     import torch
 
-    from quail_amd.engine import Engine, gemm_config
+    from quail_amd.engine import Engine, gemm_tiles
     from quail_amd.model import quantize_blocks
 
     eng = Engine(None, num_q_heads=1, num_kv_heads=1, head_dim=128, rotary=None)
@@ -234,7 +234,7 @@ def gemm_alone(reps: int = 20, seed: int = 0):
         tflops = 2.0 * m * n * k / (us * 1e-6) / 1e12
         shapes[f"{k}x{n}"] = dict(us=round(us, 2), tflops=round(tflops, 1),
                                   frac=round(tflops * 1e12 / PEAK_FP8, 4),
-                                  config=gemm_config(n, k, m))
+                                  config=gemm_tiles(n, k, m))
         del x, q, s, w, sw, out
     total_flops = sum(2.0 * m * n * k for k, n in GEMM_ALONE_SHAPES)
     total_us = sum(v["us"] for v in shapes.values())

@@ -54,8 +54,9 @@ int qx_device_is_gfx950(void);
  * Replaces Engine.gemm -> DeepGEMM fp8_gemm_nt((A, sA), (W, sW), C)
  * (quail/backends/quail/executor/attention.py:479-490); weight scales are the
  * checkpoint's weight_scale_inv (attention.py:471-477).
- * K and N multiples of 128. config selects the tile shape, tokens x weights,
- * all with two pipeline stages of one 128-K scale block each:
+ * K and N multiples of 128. config selects the tile shape, tokens x weights;
+ * 10 to 31 have two pipeline stages of one 128-K scale block each, 40 to 47 a
+ * ring of three or four stages of one, two or four blocks:
  * 10: 256x256 tiles, 8 waves, one workgroup per tile (N a multiple of 256);
  * 11: 256x128 tiles, 4 waves (any N);
  * 12: 256x320 tiles, 8 waves (N a multiple of 320: whole waves of tiles on

@@ -571,8 +571,7 @@ __global__ __launch_bounds__(HPB * QSUB * 64, 8 / (HPB * QSUB)) void paged_atten
   // MFMAs in one group ahead of the softmax: 1024-token documents 241 ->
   // 233 / 240 -> 243 us, 2048 373 -> 356 / 374 -> 360, 4096 630 -> 602 /
   // 617 -> 600, 8000 1112 -> 1076 / 1086 -> 1053; one of 700 tokens 24.7 ->
-  // 22.4 / 30.8 -> 29.6. On the longest packs the cycles fell by 18% and the
-  // time by 10%: the clock falls (1.84 to 1.68 GHz) as the step gets denser.
+  // 22.4 / 30.8 -> 29.6.
   using PV = std::conditional_t<VBF, v8bf, v8h>;
   auto read_k = [&](const uint8_t* kl, int c, v8s (&f)[2]) {
 #pragma unroll
@@ -986,7 +985,8 @@ constexpr double kShortItemTiles = 40.0;
 constexpr double kHalfEmptyTiles = 1.7;
 //   - when the 64-row workgroups do not outnumber the CUs: the 32-row ones
 //     then spread one sequence over twice as many. One document of 700
-//     tokens 22.3 us against 29.7, of 2000 tokens 58.7 against 68.8.
+//     tokens 22.3 us against 29.7, of 2000 tokens 58.7 against 68.8. (The
+//     MI355X's CUs: the rule runs on the host, without a device.)
 constexpr int64_t kCus = 256;
 
 }  // namespace

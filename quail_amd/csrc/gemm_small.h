@@ -8,13 +8,19 @@
 // 10 tiles: 10 of 256 CUs read 25 MB of weights, 97 us where the bytes take
 // 5. Smaller tiles put every CU to work; then a tile's time is its chain of
 // K blocks (76 of them): a barrier, the fragments' LDS reads (a 64 x 64 tile
-// reads 48 KiB of fragments for 16 KiB of operands) and the direct loads,
-// measured 0.17 (16 x 32) to 0.98 us (256 x 128) a block with one workgroup
-// per CU. With every operand already in L2 the mid tiles run only 5-15%
-// faster, and a copy of the loads alone draws 120 GB/s per CU from L2 where
-// the tiles draw 41-61, so it is this loop and not the memory that they wait
-// for; the 76 gate_up tiles of 256 weight rows are the exception (12 us with
-// the weights in L2, 23 without).
+// reads 48 KiB of fragments for 16 KiB of operands), the MFMAs and the direct
+// loads, measured 0.17 (16 x 32) to 0.98 us (256 x 128) a block with one
+// workgroup per CU. The reads and the MFMAs run one after the other: the next
+// block's scales are multiplied as they are read, ahead of the current
+// block's MFMAs, and LDS reads return in order, so a wave waits for most of
+// the next block's reads first (s_waitcnt lgkmcnt(5) and (2) of 19 reads on
+// 256 x 128 and 128 x 256, of 13 on 192 x 64; (10) of 14 on 64 x 64, where
+// the scales come early). A 128 x 256 block reads 128 KiB, about 0.5 us, and
+// has 0.5 us of MFMAs in its measured 1.0-1.4. Memory is not what they wait
+// for: with every operand already in L2 the mid tiles run only 5-15% faster,
+// and a copy of the loads alone draws 120 GB/s per CU from L2 where the tiles
+// draw 41-61; the 76 gate_up tiles of 256 weight rows are the exception (12
+// us with the weights in L2, 23 without).
 //   46 rows, K = 9728, N = 2560:  97 -> 14.5 us (16 x 32 tiles)
 //   333 rows, same:               98 -> 25 us (64 x 64)
 //   1003 rows, same:              98 -> 44 us (192 x 64)
@@ -90,8 +96,9 @@ struct RingCfg {
 // One workgroup per tile. Operands go memory -> LDS by direct loads the
 // compiler does not track (its own waits would drain the ring), rows of 128
 // bytes with chunk c at position c ^ (row % 8). KPB blocks share one
-// barrier: behind it the next group's fragments are read into registers
-// while the current group's MFMAs run, and the stage just left is refilled.
+// barrier: behind it the next group's fragments are read into registers, the
+// current group's MFMAs run (behind most of those reads: see above), and the
+// stage just left is refilled.
 // Two or four blocks per barrier on the small tiles, whose block is shorter
 // than a barrier's skew (16 x 32 with four: 16.3 -> 14.1 us at K = 9728);
 // the wide tiles have neither the LDS nor the need.

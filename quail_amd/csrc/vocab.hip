@@ -74,10 +74,12 @@ __device__ __forceinline__ void load_slab(const uint16_t* __restrict__ g, int64_
 // columns of their rows kept to a part of the memory channels (37 tokens,
 // V = 151936: 259 -> 218 us, 4.8 -> 5.7 TB/s; at 2560 and 5120, whose rows
 // spread over the channels by themselves, no change). Three stages; two, and
-// so two workgroups a CU at TM = 4, where several token blocks share each
-// head block and the launch waits for the L2 and the matrix cores more than
-// for memory (300 tokens: 833 -> 704 us; 128 tokens, one block, at hidden
-// 2560: three stages 203 us, two 214). The MFMA fragment of k-step s for lane half hh is K
+// so two workgroups a CU at TM = 4, where there are several token blocks (300
+// tokens at hidden 4096: 833 -> 704 us; 128 tokens, one block, at hidden 2560:
+// three stages 203 us, two 214). Such a launch goes through the whole head
+// once per token block (head blocks are the faster grid dimension, and the
+// head is larger than the caches): the 704 us are three reads of 1.24 GB at
+// 5.3 TB/s. The MFMA fragment of k-step s for lane half hh is K
 // elements [32 hh + 8 s, +8) of the chunk (16-byte chunk 4 hh + s), the
 // same permutation for both operands.
 template <int TM, int kStages>

@@ -333,9 +333,10 @@ class Engine:
         return (self.gemm_launches - 1) % self.gemm_timer_every == 0
 
     def gate_up_activation_quant(self, q_input, input_scale, linear):
-        """The gate_up projection and the quantized SiLU-gated product in one
-        launch: `activation_quant(gemm(q_input, input_scale, linear))`
-        (qwen3.py:66-67), bit for bit, without writing the bf16 gate_up rows.
+        """The gate_up projection and the quantized SiLU-gated product without
+        the bf16 gate_up rows in memory: `activation_quant(gemm(q_input,
+        input_scale, linear))` (qwen3.py:66-67), bit for bit, in one launch or
+        two (swiglu_launches).
         `linear` is the checkpoint's gate_up projection as it is."""
         w = linear.weight
         sw = self.weight_scale(linear)
