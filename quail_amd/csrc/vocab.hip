@@ -14,8 +14,8 @@
 //     to a per-token (max, sum of exp) partial; the waves' partials merge
 //     in LDS into one per (head-row block, token). The lane holding a target
 //     id's logit writes it.
-//   * vocab_finish_kernel: a workgroup of 8 waves per token merges the
-//     blocks' partials into the logsumexp (the waves' through LDS) and
+//   * vocab_finish_kernel: a workgroup per token, of one wave or 8, merges
+//     the blocks' partials into the logsumexp (the waves' through LDS) and
 //     subtracts it from the target logits.
 // The head (V x H bf16, 778 MB for Qwen3) is read once per 128 tokens, so a
 // launch over a pack's final rows is bound by streaming it from HBM.
@@ -205,9 +205,11 @@ __global__ __launch_bounds__(256) void vocab_lse_kernel(
 // One workgroup per token. A thread's partials are loaded before any is
 // merged: their addresses are known at once, and merging each as it came
 // made every one of one wave's 19 loads a memory round trip of its own (37
-// tokens at Qwen3's vocabulary: 14.0 -> 5.6 us).
-constexpr int kFinishThreads = 512;
-
+// tokens at Qwen3's vocabulary: 14.0 -> 5.6 us). A wave where it has at most
+// two rounds of loads (512 blocks), 8 waves above: 37 tokens at hidden 64, 512
+// against 64 threads, vocabulary 1000 7.3 / 6.8 us, 32,000 7.9 / 7.3, 64,000
+// 8.9 / 8.9, 151,936 15.2 / 16.5 (both launches).
+template <int kFinishThreads>
 __global__ __launch_bounds__(kFinishThreads) void vocab_finish_kernel(
     const float2* __restrict__ part, int nblk, const float* __restrict__ tlogit, int t,
     float* __restrict__ out, int64_t out_ld, int n, int tok0) {
@@ -305,11 +307,17 @@ int vocab_run(const void* normed, int64_t n_ld, const void* head, int64_t h_ld,
     if (e != hipSuccess) return (int)e;
   }
   // launches of fewer than 2^32 threads: past that the grid wraps around
-  constexpr int64_t kMaxTokens = (1LL << 31) / kFinishThreads;
-  for (int64_t tok = 0; tok < n; tok += kMaxTokens)
-    hipLaunchKernelGGL(vocab_finish_kernel, dim3((unsigned)std::min(n - tok, kMaxTokens)),
-                       dim3(kFinishThreads), 0, stream, part, nblk, tlogit, (int)t, out, out_ld,
-                       (int)n, (int)tok);
+  constexpr int64_t kMaxTokens = (1LL << 31) / 512;
+  const bool one_wave = nblk <= 512;
+  for (int64_t tok = 0; tok < n; tok += kMaxTokens) {
+    const dim3 toks((unsigned)std::min(n - tok, kMaxTokens));
+    if (one_wave)
+      hipLaunchKernelGGL(vocab_finish_kernel<64>, toks, dim3(64), 0, stream, part, nblk, tlogit,
+                         (int)t, out, out_ld, (int)n, (int)tok);
+    else
+      hipLaunchKernelGGL(vocab_finish_kernel<512>, toks, dim3(512), 0, stream, part, nblk, tlogit,
+                         (int)t, out, out_ld, (int)n, (int)tok);
+  }
   QX_LAUNCH_STATUS();
 }
 

@@ -45,7 +45,7 @@ def _close(got, want, target_logits):
 @pytest.mark.parametrize("n,vocab,hidden", [(1, 151936, 2560), (37, 151936, 2560),
                                             (100, 151936, 2560), (300, 4096, 256),
                                             (64, 1000, 128), (130, 1000, 64),
-                                            (20, 700, 192)])
+                                            (20, 700, 192), (37, 65536, 64), (37, 65537, 64)])
 def test_vocab_logprobs_match_float64(n, vocab, hidden):
     normed, head = _case(n, vocab, hidden, seed=n + vocab)
     targets = [0, 11, vocab // 2, vocab - 1, 11]
