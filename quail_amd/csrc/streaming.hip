@@ -235,11 +235,18 @@ __global__ __launch_bounds__(64 * WPR) void norm_quant_row_kernel(
 // 103.0; MODE 1, hidden 2560: 333 5.2 -> 3.9, 2048 6.5 -> 7.8, 16384 27.1 ->
 // 35.5; hidden 5120: 16384 54.7 -> 59.4; hidden 8192: 16384 134 -> 112; MODE
 // 2, hidden 2560: 333 5.6 -> 4.1, 4096 12.6 -> 13.6; hidden 5120: 16384 106.5
-// -> 86.5; hidden 128: 2.8 -> 2.9 at any few rows.
+// -> 86.5; hidden 128: 2.8 -> 2.9 at any few rows. The line for few rows, MODE
+// 1, at 1280 / 1408 / 1536 rows: 2 passes (hidden 1024) 3.41 -> 3.38, 3.42 ->
+// 3.55, 3.44 -> 3.59; 5 (2560) 5.61 -> 5.01, 5.63 -> 5.94, 5.68 -> 6.04; 6
+// (3072) 6.28 -> 5.43, 6.41 -> 6.50, 6.43 -> 6.65; 7 (3584) 7.08 -> 6.71, 7.28
+// -> 7.34, 7.31 -> 7.51; 3, 4 and 8 passes 1-9% faster at all three, and so
+// MODE 2 but for 2 and 5 passes at 1536 (4.00 -> 4.09, 6.98 -> 7.22), MODE 0
+// 5-12% at 1536.
 constexpr bool always_row_workgroups(int niter, int mode) { return niter > (mode == 1 ? 10 : 8); }
 constexpr bool never_row_workgroups(int niter) { return niter < 2; }
 bool row_workgroups(int niter, int mode, int n) {
-  return n <= 1536 || (mode == 0 && niter >= 5 && n >= 4096);
+  const bool early = mode == 1 && (niter == 2 || (niter >= 5 && niter <= 7));
+  return n <= (early ? 1280 : 1536) || (mode == 0 && niter >= 5 && n >= 4096);
 }
 
 // One workgroup per row, in launches of fewer than 2^32 threads (more are
