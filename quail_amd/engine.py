@@ -53,19 +53,19 @@ GEMM_ODD_WIDTH_CONFIG = 11
 CUS = 256
 
 
-_Environ = type(os.environ)
+_Environ = type(os.environ) if os.name == "posix" else None   # its dict's keys are bytes
 
 
 def _forced(name):
     """os.environ.get(name) of what os.environ is at the call. Each GEMM asks,
     and Python's own environment mapping raises and catches KeyError for every
-    name that is not set (0.9 us against 0.4): its dict is asked instead,
+    name that is not set (0.6 us against 0.26): its dict is asked instead,
     where it has one. Any other mapping in its place is asked as it is."""
     env = os.environ
     data = getattr(env, "_data", None) if type(env) is _Environ else None
     if type(data) is not dict:
         return env.get(name)
-    value = data.get(env.encodekey(name))
+    value = data.get(name.encode())
     return None if value is None else env.decodevalue(value)
 
 
